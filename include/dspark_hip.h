@@ -464,6 +464,13 @@ int dsk_logits_penalize(float* logits, int64_t ldl, int R, const int32_t* row_pt
 int dsk_row_logprobs(const float* logits, int64_t ldl, int R, int64_t V, const int32_t* tokens,
                      int top_k, float* chosen, int32_t* top_ids, float* top_vals, dsk_stream_t stream);
 
+/* The same with scratch: every row is split over workgroups (V <= 2^19, R <= 65535).
+ * dsk_row_logprobs_ws_bytes returns 0 for shapes it does not take (use dsk_row_logprobs). */
+size_t dsk_row_logprobs_ws_bytes(int R, int64_t V, int top_k);
+int dsk_row_logprobs_ws(const float* logits, int64_t ldl, int R, int64_t V, const int32_t* tokens,
+                        int top_k, float* chosen, int32_t* top_ids, float* top_vals, void* workspace,
+                        size_t ws_bytes, dsk_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -90,6 +90,9 @@ SIGNATURES: dict[str, tuple] = {
                                  c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "dsk_row_logprobs": (c_int, [c_void_p, c_int64, c_int, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                  c_void_p]),
+    "dsk_row_logprobs_ws_bytes": (c_size_t, [c_int, c_int64, c_int]),
+    "dsk_row_logprobs_ws": (c_int, [c_void_p, c_int64, c_int, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                    c_void_p, c_size_t, c_void_p]),
     "dsk_logits_penalize": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
 }
 

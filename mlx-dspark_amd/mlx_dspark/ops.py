@@ -605,6 +605,12 @@ def row_logprobs(logits: torch.Tensor, tokens: torch.Tensor, top_k: int = 0):
     chosen = torch.empty(R, dtype=torch.float32, device=dev)
     ids = torch.empty((R, max(top_k, 1)), dtype=torch.int32, device=dev)
     vals = torch.empty((R, max(top_k, 1)), dtype=torch.float32, device=dev)
-    call("dsk_row_logprobs", ptr(logits), logits.stride(0), R, V, ptr(tokens), int(top_k), ptr(chosen), ptr(ids),
-         ptr(vals), stream_ptr())
+    need = _hip.lib.dsk_row_logprobs_ws_bytes(R, V, int(top_k))
+    if need == 0:   # shapes beyond the split form (or arguments the entry refuses)
+        call("dsk_row_logprobs", ptr(logits), logits.stride(0), R, V, ptr(tokens), int(top_k), ptr(chosen), ptr(ids),
+             ptr(vals), stream_ptr())
+    else:
+        buf = torch.empty(need, dtype=torch.uint8, device=dev)   # per call: rows may be scored on any stream
+        call("dsk_row_logprobs_ws", ptr(logits), logits.stride(0), R, V, ptr(tokens), int(top_k), ptr(chosen),
+             ptr(ids), ptr(vals), ptr(buf), need, stream_ptr())
     return chosen, ids[:, :top_k], vals[:, :top_k]
