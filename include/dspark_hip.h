@@ -305,6 +305,14 @@ int dsk_qkv_rope_append_rn(const void* qkv, int qkv_splits, int B, int W, int nq
                            uint32_t* k_sb, uint32_t* v_sb, uint16_t* q_out, const float* x_ssq,
                            int x_tiles, float x_eps, dsk_stream_t stream);
 
+/* dsk_attention for the many rows of a prompt (head_dim 128 or 256, no soft-cap, at most 1024 pages per
+ * row, row-major output), with the probabilities carried as three bf16 terms (within 2^-26) as in the
+ * verify kernels; dsk_attention's own many-query pass carries two (2^-17). No workspace. */
+int dsk_attention_rows(const uint16_t* q, int B, int W, int nq, int nkv, int hd, float scale, int causal,
+                       int window, const int32_t* seq_lens, const int32_t* block_table, int max_pages,
+                       int page, int kv_dtype, const void* k_pool, const void* v_pool, const uint32_t* k_sb,
+                       const uint32_t* v_sb, uint16_t* out, dsk_stream_t stream);
+
 /* dsk_qkv_rope_append followed by dsk_attention in one kernel (plus the split combine):
  * from the qkv projection (bf16 or fp32 split-K slices, as for dsk_qkv_rope_append, with
  * pos_offset 0) each workgroup forms its queries (q RMSNorm, RoPE at seq_lens[b] + i); the
@@ -454,6 +462,25 @@ int dsk_markov_block(const float* base, int64_t ldb, int B, int cap, int64_t V, 
  * plus each row's draft prefix. */
 int dsk_logits_penalize(float* logits, int64_t ldl, int R, const int32_t* row_ptr,
                         const int32_t* ids, const float* vals, dsk_stream_t stream);
+
+/* Products of any number of rows (prompts, drafter contexts).
+ * dsk_rows_prep, one pass over the rows h [M][K] (bf16, row stride ldh): h = bf16(h + y) when y is
+ * given (y RMSNorm-ed with y_norm_w first when that is given: the sandwich norm), copy = h (tap);
+ * then, when x is given, the product's input: h itself (norm_w null), bf16(h * rsqrt(mean(h^2) + eps)
+ * * norm_w), or with later != 0 bf16(h * norm_w) and rsc[m] = rsqrt(mean(h^2) + eps). x and xt (the
+ * sums of x over each 64 columns, as three bf16 terms) are in dsk_w8_rows' operand order:
+ * ceil16(M) * K values, and 3 * ceil16(M) * Gp with Gp = K / 64 rounded up to 64.
+ * dsk_w8_rows: x [M][K] . deq(W)^T over tiled codes (bits 8 or 4), row m scaled by rsc[m] when given:
+ * DSK_EPI_STORE y [M][N] bf16; SWIGLU / GEGLU (paired W) y [M][N / 2] bf16; RESIDUAL h = bf16(h + .)
+ * in place and copy = h. K % 256 == 0, N % 16 == 0. Replaces the projections of the reference's
+ * chunked prefill (src/mlx_dspark/generate.py:613-656) and context ingest
+ * (src/mlx_dspark/model.py:247-256). */
+int dsk_rows_prep(uint16_t* h, int64_t ldh, const uint16_t* y, int64_t ldy, const uint16_t* y_norm_w,
+                  uint16_t* copy, int64_t ldc, int M, int64_t K, const uint16_t* norm_w, int later,
+                  float eps, uint16_t* x, uint16_t* xt, float* rsc, dsk_stream_t stream);
+int dsk_w8_rows(const uint16_t* x, const uint16_t* xt, const uint8_t* wt, const uint32_t* sb, int bits,
+                int M, int64_t N, int64_t K, int epi, const float* rsc, uint16_t* y, int64_t ldy,
+                uint16_t* h, int64_t ldh, uint16_t* copy, int64_t ldc, dsk_stream_t stream);
 
 /* Per-token log-probabilities of committed tokens (OpenAI logprobs): for each row r of
  * logits [R][V] (row stride ldl, fp32), lse = max + log(sum exp(x - max)) (the raw target

@@ -1284,33 +1284,29 @@ __global__ __launch_bounds__(kVerifyCombineThreads) void attention_verify_combin
 }
 
 // ----------------------------------------------------------------------------- many-query pass
-// A prefill (head_dim 128, more than 64 new tokens per row): one workgroup per (row b, kv head,
-// block of 128 query rows), no key splits and so no combine. The row block's keys stream through
+// A prompt pass (head_dim 128 or 256, more than 64 new tokens per row): one workgroup per (row b, kv
+// head, block of query rows), no key splits and so no combine. The row block's keys stream through
 // LDS in 64-key blocks (double-buffered: block n + 1 is dequantised into the other buffer while
-// block n is scored, block n + 2's loads are in flight meanwhile, one barrier per block). Each
-// of the kPfWaves waves owns two 16-query tiles, so every K and V fragment it reads from LDS
-// feeds two tiles' MFMAs, and each block's dequantisation is shared by all the rows. The row
+// block n is scored, block n + 2's loads are in flight meanwhile, one barrier per block). Each of the
+// NW waves owns TPW 16-query tiles, so every K and V fragment it reads from LDS feeds TPW tiles'
+// MFMAs, and each block's dequantisation is shared by all the rows. The row
 // sums of P come out of the P.V MFMAs as one more V^T tile of ones. Scores S^T = K . Q^T and O^T = V^T . P^T as in the other attention kernels; masking
 // runs only on blocks that straddle a wave's causal diagonal, its window edge or the last key.
 // Row blocks with the most keys are launched first (the grid's y runs from the last block).
 constexpr int kPfKeys = 64;                   // keys per LDS block
-constexpr int kPfKRow = 128 + 8;              // K rows in LDS (bf16, padded: conflict-free reads)
 constexpr int kPfVRow = kPfKeys + 8;          // V^T rows in LDS (bf16, padded)
-constexpr int kPfTiles = 2;                   // 16-query tiles per wave
-#ifndef DSK_PF_WAVES
-#define DSK_PF_WAVES 8
-#endif
-constexpr int kPfWaves = DSK_PF_WAVES;
-constexpr int kPfThreads = kPfWaves * 64;
-constexpr int kPfRows = kPfWaves * kPfTiles * 16;  // query rows per workgroup
 constexpr int kPfMaxPages = 1024;             // page ids of a row block's keys held in LDS
 
-// At most 256 VGPRs (two waves per SIMD: one 8-wave workgroup per CU, whose waves' staging and
-// MFMAs interleave). On the 4096-token Qwen3-8B layer: 436 us with 4 waves and no bound, 299 us
-// with 4 waves and this bound, 239 us with 8 waves sharing each block's dequantisation.
-template <int KVT>
-__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prefill_kernel(AttnArgs a) {
-  constexpr int HD = 128, KS = HD / 32, DT = HD / 16, NKT = kPfKeys / 16, TPW = kPfTiles, NTHR = kPfThreads;
+// Shapes: 8 waves of two tiles at head_dim 128 (256 rows; at most 256 VGPRs, two waves per SIMD, whose
+// staging and MFMAs interleave). On the 4096-token Qwen3-8B layer: 436 us with 4 waves and no bound, 299 us
+// with 4 waves and this bound, 239 us with 8 waves sharing each block's dequantisation (one bf16 term
+// of P). 4 waves of one tile where the 256-row blocks leave CUs idle, and at head_dim 256, where the
+// two K/V buffers fill the LDS.
+template <int HD, int KVT, int TERMS, int NW, int TPW>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, 2))) void attention_prefill_kernel(AttnArgs a) {
+  constexpr int KS = HD / 32, DT = HD / 16, NKT = kPfKeys / 16, NTHR = NW * 64;
+  constexpr int kPfKRow = HD + 8;         // K rows in LDS (bf16, padded: conflict-free reads)
+  constexpr int kPfRows = NW * TPW * 16;  // query rows per workgroup
   constexpr int CK = kPfKeys * (HD / 8) / NTHR;        // 8-dim K chunks per thread
   constexpr int CV = (kPfKeys / 2) * (HD / 8) / NTHR;  // (2 keys x 8 dims) V chunks per thread
   static_assert(CK * NTHR == kPfKeys * (HD / 8) && CV * NTHR == (kPfKeys / 2) * (HD / 8), "whole chunks per thread");
@@ -1495,25 +1491,27 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         for (int d = 0; d < DT; ++d) o[t][d] *= alpha;
       }
     }
-    // ---- O^T[d][q] += V^T . P^T with P as hi + lo (two MFMAs per fragment and tile; a prefill
-    // is MFMA-heavy, so the third term of the verify kernels is left out: P within 2^-17):
-    // each V^T fragment feeds both query tiles
+    // ---- O^T[d][q] += V^T . P^T with P as TERMS bf16 terms, an MFMA per term, fragment and tile (two:
+    // hi + lo, P within 2^-17; three: 2^-26): each V^T fragment feeds all query tiles
     const uint16_t* vt16 = reinterpret_cast<const uint16_t*>(vt[buf]);
 #pragma unroll
     for (int cp = 0; cp < NKT / 2; ++cp) {
-      bf16x8 pk[TPW][2];
+      bf16x8 pk[TPW][TERMS];
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
-        uint32_t w[2][4];
+        uint32_t w[TERMS][4];
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) {
             const f32x4& pv = st[t][2 * cp + u];
-            split2_bf16x2(pv[2 * hh], pv[2 * hh + 1], w[0][2 * u + hh], w[1][2 * u + hh]);
+            uint32_t tt[TERMS];
+            split_terms_bf16x2<TERMS>(pv[2 * hh], pv[2 * hh + 1], tt);
+#pragma unroll
+            for (int k = 0; k < TERMS; ++k) w[k][2 * u + hh] = tt[k];
           }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) pk[t][k] = __builtin_bit_cast(bf16x8, (u32x4{w[k][0], w[k][1], w[k][2], w[k][3]}));
+        for (int k = 0; k < TERMS; ++k) pk[t][k] = __builtin_bit_cast(bf16x8, (u32x4{w[k][0], w[k][1], w[k][2], w[k][3]}));
       }
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
@@ -1522,12 +1520,12 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2
         const uint2 hi = *reinterpret_cast<const uint2*>(vr + 16);
         const bf16x8 vf = __builtin_bit_cast(bf16x8, (u32x4{lo.x, lo.y, hi.x, hi.y}));
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
+        for (int k = 0; k < TERMS; ++k)
 #pragma unroll
           for (int t = 0; t < TPW; ++t) o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pk[t][k], o[t][d], 0, 0, 0);
       }
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < TERMS; ++k)
 #pragma unroll
         for (int t = 0; t < TPW; ++t) lt[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pk[t][k], lt[t], 0, 0, 0);
     }
@@ -1587,6 +1585,26 @@ static void launch_attention(const AttnArgs& a, int kv_dtype, bool softcap, dim3
   }
 }
 
+// many-query passes (prompts): whole key ranges per query block, no splits, no combine
+template <int HD, int TERMS, int NW, int TPW>
+static void launch_prompt_shape(const AttnArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(a.B * a.nkv), (unsigned)ceil_div(a.R, NW * TPW * 16)), blk(NW * 64);
+  if (a.kv_dtype == DSK_KV_U8)
+    hipLaunchKernelGGL((attention_prefill_kernel<HD, DSK_KV_U8, TERMS, NW, TPW>), grid, blk, 0, st, a);
+  else
+    hipLaunchKernelGGL((attention_prefill_kernel<HD, DSK_KV_BF16, TERMS, NW, TPW>), grid, blk, 0, st, a);
+}
+template <int TERMS>
+static void launch_prompt_attention(AttnArgs& a, int hd, hipStream_t st) {
+  a.nsplit = 1;
+  a.part_o = nullptr;
+  a.part_ml = nullptr;
+  if constexpr (TERMS == 3)
+    if (hd == 256) return launch_prompt_shape<256, TERMS, 4, 1>(a, st);
+  if ((int64_t)a.B * a.nkv * ceil_div(a.R, 256) < 256) return launch_prompt_shape<128, TERMS, 4, 1>(a, st);
+  launch_prompt_shape<128, TERMS, 8, 2>(a, st);
+}
+
 // Keys of one LDS block; a split streams nblk blocks (graph-stable: the split grid depends on
 // max_ctx only). One block per split gives the most splits, which sizes the workspace.
 static int attn_split_keys(int hd, int) {
@@ -1639,14 +1657,7 @@ static int attention_run(AttnArgs& a, int hd, int max_ctx, float softcap, void* 
   a.fused = fused ? 1 : 0;
   const bool sc = softcap > 0.0f;
   if (hd == 128 && !fused && !sc && !a.out_packed && a.W > kAttnVerifyMaxW && a.max_pages <= kPfMaxPages) {
-    // many-query passes (prefills): whole key ranges per query block, no splits, no combine
-    a.nsplit = 1;
-    a.kps = max_ctx;
-    a.part_o = nullptr;
-    a.part_ml = nullptr;
-    const dim3 pgrid((unsigned)(a.B * a.nkv), (unsigned)ceil_div(a.R, kPfRows));
-    if (a.kv_dtype == DSK_KV_U8) hipLaunchKernelGGL(attention_prefill_kernel<DSK_KV_U8>, pgrid, dim3(kPfThreads), 0, st, a);
-    else hipLaunchKernelGGL(attention_prefill_kernel<DSK_KV_BF16>, pgrid, dim3(kPfThreads), 0, st, a);
+    launch_prompt_attention<2>(a, hd, st);
     DSK_LAUNCH_CHECK(who);
     return DSK_OK;
   }
@@ -1893,6 +1904,44 @@ extern "C" int dsk_attention(const uint16_t* q, int B, int W, int nq, int nkv, i
   a.out = out;
   a.out_packed = out_packed ? 1 : 0;
   return attention_run(a, hd, max_ctx, softcap, workspace, ws_bytes, false, as_stream(stream), "dsk_attention");
+}
+
+extern "C" int dsk_attention_rows(const uint16_t* q, int B, int W, int nq, int nkv, int hd, float scale, int causal,
+                                  int window, const int32_t* seq_lens, const int32_t* block_table, int max_pages,
+                                  int page, int kv_dtype, const void* k_pool, const void* v_pool, const uint32_t* k_sb,
+                                  const uint32_t* v_sb, uint16_t* out, dsk_stream_t stream) {
+  const char* who = "dsk_attention_rows";
+  DSK_REQUIRE(q && seq_lens && block_table && k_pool && v_pool && out, "%s: null pointer", who);
+  DSK_REQUIRE(hd == 128 || hd == 256, "%s: head_dim %d not supported (128, 256)", who, hd);
+  DSK_REQUIRE(B > 0 && W > 0 && nq > 0 && nkv > 0 && nq % nkv == 0 && page > 0, "%s: bad shape", who);
+  DSK_REQUIRE(kv_dtype == DSK_KV_BF16 || (kv_dtype == DSK_KV_U8 && k_sb && v_sb), "%s: u8 KV needs sb", who);
+  DSK_REQUIRE(max_pages > 0 && max_pages <= kPfMaxPages, "%s: %d pages per row (at most %d)", who, max_pages,
+              kPfMaxPages);
+  DSK_REQUIRE((int64_t)W * (nq / nkv) <= 65535 * 64, "%s: W=%d", who, W);
+  AttnArgs a = {};
+  a.q = q;
+  a.B = B;
+  a.W = W;
+  a.nq = nq;
+  a.nkv = nkv;
+  a.G = nq / nkv;
+  a.R = W * a.G;
+  a.scale = scale;
+  a.causal = causal;
+  a.window = window;
+  a.seq_lens = seq_lens;
+  a.block_table = block_table;
+  a.max_pages = max_pages;
+  a.page = page;
+  a.kv_dtype = kv_dtype;
+  a.k_pool = const_cast<void*>(k_pool);
+  a.v_pool = const_cast<void*>(v_pool);
+  a.k_sb = const_cast<uint32_t*>(k_sb);
+  a.v_sb = const_cast<uint32_t*>(v_sb);
+  a.out = out;
+  launch_prompt_attention<3>(a, hd, as_stream(stream));
+  DSK_LAUNCH_CHECK(who);
+  return DSK_OK;
 }
 
 extern "C" int dsk_qkv_attention(const void* qkv, int qkv_splits, int B, int W, int nq, int nkv, int hd,

@@ -2,6 +2,7 @@
 // library GEMM of a long prompt), and the row-wise RMSNorm and gated activations that sit between
 // those GEMMs. Every kernel works on plain row-major bf16 [M, K] activations of any row count.
 #include "common.h"
+#include "wfrag.h"
 
 namespace dsk {
 
@@ -101,12 +102,6 @@ __global__ __launch_bounds__(kRowThreads) void rows_rmsnorm_kernel(const uint16_
   }
 }
 
-__device__ __forceinline__ float silu_r(float g) { return g / (1.0f + expf(-g)); }
-__device__ __forceinline__ float gelu_tanh_r(float x) {
-  const float c = 0.7978845608028654f;  // sqrt(2/pi)
-  return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
-}
-
 // out[m][i] = bf16(bf16(act(gate[m][i])) * up[m][i]) with gate = gu[m][i], up = gu[m][I + i]
 // (bf16 projections; act = SiLU or tanh-GeLU), as the GEMM's gated epilogue computes it.
 template <bool GELU>
@@ -124,7 +119,7 @@ __global__ __launch_bounds__(256) void rows_gated_kernel(const uint16_t* __restr
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float gb = bf16_to_f32(g[e]);
-    const float act = round_bf16(GELU ? gelu_tanh_r(gb) : silu_r(gb));
+    const float act = round_bf16(GELU ? gelu_tanh_f(gb) : silu_f(gb));
     o[e] = f32_to_bf16(act * bf16_to_f32(u[e]));
   }
   *reinterpret_cast<u32x4*>(out + m * ldo + i) = *reinterpret_cast<const u32x4*>(o);

@@ -64,6 +64,8 @@ SIGNATURES: dict[str, tuple] = {
     "dsk_attention": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_float,
                               c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
                               c_void_p, c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
+    "dsk_attention_rows": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
+                                   c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "dsk_qkv_attention": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float,
                                   c_void_p, c_float, c_int, c_int, c_float, c_void_p, c_int, c_void_p, c_int, c_int,
                                   c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_size_t,
@@ -90,6 +92,10 @@ SIGNATURES: dict[str, tuple] = {
                                  c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "dsk_row_logprobs": (c_int, [c_void_p, c_int64, c_int, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                  c_void_p]),
+    "dsk_rows_prep": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int64, c_void_p,
+                              c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "dsk_w8_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int, c_void_p,
+                            c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "dsk_row_logprobs_ws_bytes": (c_size_t, [c_int, c_int64, c_int]),
     "dsk_row_logprobs_ws": (c_int, [c_void_p, c_int64, c_int, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_size_t, c_void_p]),

@@ -18,7 +18,7 @@ import torch
 
 from . import ops
 from .kv import PagedKVCache
-from .qwen3 import MAX_ROWS
+from .qwen3 import MAX_ROWS, PREFILL_CHUNK
 
 
 def ingest_context(d, target_hidden: torch.Tensor, cache: PagedKVCache, n_valid=None) -> None:
@@ -37,8 +37,13 @@ def ingest_context(d, target_hidden: torch.Tensor, cache: PagedKVCache, n_valid=
         raise ValueError("a device-counted context append must fit one pass")
     cache.check_room(S + c.block_size)
     H = c.hidden_size
-    for r0 in range(0, S, MAX_ROWS):
-        r1 = min(S, r0 + MAX_ROWS)
+    r1 = 0
+    while r1 < S:
+        r0, r1 = r1, min(S, r1 + PREFILL_CHUNK)
+        if r1 - r0 > MAX_ROWS and _rows_ok(d):
+            _ingest_many(d, th[r0:r1], cache, v_norm)
+            continue
+        r1 = min(r1, r0 + MAX_ROWS)
         hcp = ops.w8_gemm(ops.pack(th[r0:r1]), d.fc, epi=ops.DSK_EPI_PARTIAL)          # fc(target_hidden)
         xc = ops.act_pack(M=r1 - r0, K=H, part=hcp, norm_w=d.hidden_norm, eps=c.rms_norm_eps)
         for l, L in enumerate(d.layers):
@@ -52,6 +57,27 @@ def ingest_context(d, target_hidden: torch.Tensor, cache: PagedKVCache, n_valid=
             cache.note_lengths([cache.lengths[0] + (r1 - r0)])
     if n_valid is not None:
         ops.lens_add(cache.seq_lens, n_valid, 1)
+
+
+def _rows_ok(d) -> bool:
+    """Whether the products of many rows take this drafter's widths (ops.rows_prep, ops.w8_rows)."""
+    return all(k % 256 == 0 and k <= ops.ROWS_MAX_K for k in (d.fc.K, d.config.hidden_size))
+
+
+def _ingest_many(d, th: torch.Tensor, cache: PagedKVCache, v_norm) -> None:
+    """Append more than MAX_ROWS context rows in one pass (ingest_context's rounding points)."""
+    c, a = d.config, d.args
+    n = th.shape[0]
+    if th.dtype != torch.bfloat16 or th.stride(-1) != 1 or th.stride(0) % 8 or th.data_ptr() % 16:
+        th = th.contiguous().to(torch.bfloat16)
+    xc = ops.rows_prep(ops.w8_rows(ops.rows_prep(th), d.fc), norm_w=d.hidden_norm, eps=c.rms_norm_eps)
+    for l, L in enumerate(d.layers):
+        k_pool, v_pool, k_sb, v_sb = cache.layer_args(l)
+        ops.qkv_rope_append(ops.w8_rows(xc, L.kv_view(d.args)), 1, n, 0, a.num_key_value_heads, a.head_dim, None,
+                            L.k_norm, c.rms_norm_eps, d.inv_freq, cache.seq_lens, cache.block_table, cache.page,
+                            cache.kv_dtype, k_pool, v_pool, k_sb, v_sb, None, v_norm=v_norm)
+    ops.lens_add(cache.seq_lens, None, n)
+    cache.note_lengths([cache.lengths[0] + n])
 
 
 def ingest_rows(d, fused: torch.Tensor, cache: PagedKVCache, n_valid: torch.Tensor) -> None:

@@ -20,8 +20,8 @@ from ._hip import (DSK_BF16, DSK_EPI_GEGLU, DSK_EPI_PARTIAL, DSK_EPI_RESIDUAL, D
 
 __all__ = [
     "W8Weight", "W8Table", "Workspace", "Packed", "act_pack", "pack", "pack_rn", "w8_gemm", "w8_residual", "w8_embed",
-    "w8_dequant", "rows_rmsnorm", "rows_gated",
-    "qkv_rope_append", "attention", "qkv_attention", "row_logprobs", "accept_greedy", "accept_sample", "sample_rows",
+    "w8_dequant", "Rows", "rows_prep", "w8_rows", "rows_rmsnorm", "rows_gated",
+    "qkv_rope_append", "attention", "attention_rows", "qkv_attention", "row_logprobs", "accept_greedy", "accept_sample", "sample_rows",
     "argmax_rows", "lens_add",
     "rope_inv_freq", "DSK_EPI_STORE", "DSK_EPI_SWIGLU", "DSK_EPI_GEGLU", "DSK_EPI_PARTIAL", "DSK_KV_BF16",
     "DSK_KV_U8",
@@ -337,6 +337,67 @@ def w8_gemm(x: Packed, w: W8Weight, *, epi: int = DSK_EPI_STORE, out=None, out_d
     return out
 
 
+@dataclass
+class Rows:
+    """An [M, K] bf16 input of w8_rows in the product's operand order, with what the product needs
+    beside it (dsk_rows_prep): the terms of its group sums and, for a norm applied later, the row
+    scales."""
+
+    data: torch.Tensor
+    xt: torch.Tensor
+    M: int
+    K: int
+    rsc: torch.Tensor | None = None
+
+
+ROWS_MAX_K = 24576   # widest rows dsk_rows_prep holds in registers
+
+
+def rows_prep(h: torch.Tensor, *, norm_w: torch.Tensor | None = None, eps: float = 0.0, later: bool = False,
+              part: torch.Tensor | None = None, part_norm_w: torch.Tensor | None = None,
+              copy: torch.Tensor | None = None, out: bool = True) -> Rows | None:
+    """The input of w8_rows over rows h [M, K] bf16 (any M): h += part first when given (in place;
+    part_norm_w: its sandwich norm), copy = h; then RMSNorm(h) with norm_w (``later``: bf16(h * w), its
+    row scale left to the product), or h itself. out=False stops after the residual add."""
+    M, K = h.shape
+    for t in (h, part, copy):
+        if t is not None and (t.dtype != torch.bfloat16 or tuple(t.shape) != (M, K) or not _rows_ok(t)):
+            raise ValueError(f"rows_prep: rows must be bf16 [{M}, {K}] with unit column stride, 16-byte aligned rows")
+    x = xt = rsc = None
+    if out:
+        Mp = (M + 15) // 16 * 16
+        x = torch.empty(Mp * K, dtype=torch.bfloat16, device=h.device)
+        xt = torch.empty(3 * Mp * ((K // 64 + 63) // 64 * 64), dtype=torch.bfloat16, device=h.device)
+        rsc = torch.empty(M, dtype=torch.float32, device=h.device) if later and norm_w is not None else None
+    call("dsk_rows_prep", ptr(h), h.stride(0), ptr(part), 0 if part is None else part.stride(0), ptr(part_norm_w),
+         ptr(copy), 0 if copy is None else copy.stride(0), M, K, ptr(norm_w if out else None), int(later),
+         float(eps), ptr(x), ptr(xt), ptr(rsc), stream_ptr())
+    return Rows(x, xt, M, K, rsc) if out else None
+
+
+def w8_rows(x: Rows, w: W8Weight, *, epi: int = DSK_EPI_STORE, h: torch.Tensor | None = None,
+            copy: torch.Tensor | None = None) -> torch.Tensor:
+    """x . deq(W)^T for any number of rows (dsk_w8_rows): bf16 [M, N]; SWIGLU / GEGLU (paired W)
+    [M, N/2]; RESIDUAL adds it to h in place (copy = h) and returns h."""
+    M, K = x.M, x.K
+    if K != w.K:
+        raise ValueError(f"w8_rows: x has K={K}, W has K={w.K}")
+    gated = epi in (DSK_EPI_SWIGLU, DSK_EPI_GEGLU)
+    if gated != w.paired:
+        raise ValueError("w8_rows: the gated epilogues, and they alone, take a paired gate|up weight")
+    y = None
+    if epi == DSK_EPI_RESIDUAL:
+        for t in (h,) if copy is None else (h, copy):
+            if tuple(t.shape) != (M, w.N) or t.dtype != torch.bfloat16 or not _rows_ok(t):
+                raise ValueError(f"w8_rows: h and copy must be bf16 [{M}, {w.N}] with aligned unit-stride rows")
+    else:
+        y = torch.empty((M, w.N // 2 if gated else w.N), dtype=torch.bfloat16, device=x.data.device)
+    call("dsk_w8_rows", ptr(x.data), ptr(x.xt), ptr(w.wt), ptr(w.sb), w.bits, M, w.N, K, int(epi),
+         ptr(x.rsc), ptr(y), 0 if y is None else y.stride(0), ptr(h if y is None else None),
+         0 if y is not None else h.stride(0), ptr(copy), 0 if copy is None else copy.stride(0), stream_ptr())
+    return h if y is None else y
+
+
 def w8_dequant(w: W8Weight, out: torch.Tensor | None = None) -> torch.Tensor:
     """bf16 [N, K] rows bf16(s * q + b) of a W8 / W4 weight in source row order (a paired
     gate|up weight: the gate rows, then the up rows), for a library GEMM over many rows."""
@@ -437,6 +498,20 @@ def attention(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page,
          ptr(buf), buf.numel(), stream_ptr())
     return out
 
+
+
+def attention_rows(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page, kv_dtype, k_pool, v_pool,
+                   k_sb=None, v_sb=None, *, causal=True, window=0):
+    """attention of a prompt's many rows, bf16 [B*W, nq*hd], with the verify kernels' float32
+    probabilities (dsk_attention_rows; dsk_attention where its shapes end)."""
+    if hd not in (128, 256) or block_table.shape[1] > 1024:
+        return attention(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page, kv_dtype, k_pool, v_pool,
+                         k_sb, v_sb, causal=causal, window=window)
+    out = torch.empty((B * W, nq * hd), dtype=torch.bfloat16, device=q.device)
+    call("dsk_attention_rows", ptr(q), B, W, nq, nkv, hd, float(scale), int(bool(causal)), int(window), ptr(seq_lens),
+         ptr(block_table), block_table.shape[1], page, kv_dtype, ptr(k_pool), ptr(v_pool), ptr(k_sb), ptr(v_sb),
+         ptr(out), stream_ptr())
+    return out
 
 
 def qkv_attention(qkv, B, W, nq, nkv, hd, q_norm, k_norm, eps, inv_freq, scale, seq_lens, max_ctx, block_table,

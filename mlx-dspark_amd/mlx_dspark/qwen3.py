@@ -298,8 +298,9 @@ class Qwen3W8:
         """Single-row prefill. Returns (last-position logits [1, 1, V], fused of the whole prompt
         [1, L, n_tap*H] or None). on_chunk(fused_chunk, pos) lets a drafter ingest the hidden
         states chunk by chunk. A Qwen3-layout prompt of DENSE_MIN_ROWS rows or more runs layer
-        by layer over all its rows (prefill_dense); shorter ones (or dense=False) in forward
-        passes of ``chunk`` rows."""
+        by layer over all its rows (prefill_dense). Others (or dense=False) run in pieces of up to
+        PREFILL_CHUNK rows whose projections keep the codes' own arithmetic (_rows_pass), with a last
+        piece of at most MAX_ROWS rows (or every piece, when ``chunk`` is smaller) in a forward pass."""
         if not torch.is_tensor(ids):
             ids = torch.tensor(ids, dtype=torch.int32)
         ids = ids.reshape(1, -1).to(self.device, torch.int32)
@@ -312,10 +313,12 @@ class Qwen3W8:
         parts = []
         out = None
         pos = cache.lengths[0]
-        for c0 in range(0, L, chunk):
-            c1 = min(L, c0 + chunk)
+        piece = PREFILL_CHUNK if chunk == MAX_ROWS and self._rows_ok else chunk
+        for c0 in range(0, L, piece):
+            c1 = min(L, c0 + piece)
             last = c1 == L
-            out, fused = self.forward(ids[:, c0:c1], cache, tap, logits="last" if last else "none")
+            run = self._rows_pass if c1 - c0 > MAX_ROWS else self.forward
+            out, fused = run(ids[:, c0:c1], cache, tap, logits="last" if last else "none")
             if fused is not None:
                 if on_chunk is not None:
                     on_chunk(fused, pos)
@@ -327,6 +330,67 @@ class Qwen3W8:
             fused_all = parts[0] if len(parts) == 1 else torch.cat(parts, dim=1)
         return out, fused_all
 
+
+    # ------------------------------------------------------------------ many rows
+    @property
+    def _rows_ok(self) -> bool:
+        """Whether _rows_pass takes this model's widths (ops.rows_prep, ops.w8_rows)."""
+        a = self.args
+        return all(k % 256 == 0 and k <= ops.ROWS_MAX_K
+                   for k in (a.hidden_size, a.num_attention_heads * a.head_dim, a.intermediate_size))
+
+    def _rows_pass(self, ids: torch.Tensor, cache: PagedKVCache, tap=None, *, logits: str = "last"):
+        """forward over one row of more than MAX_ROWS new tokens, with its rounding points: row-major
+        activations between the products of many rows. logits: "last" or "none"; advances the cache.
+        Returns (logits [1, 1, V] or None, fused [1, L, n_tap*H] or None)."""
+        a = self.args
+        L, H, eps = ids.shape[1], a.hidden_size, a.rms_norm_eps
+        nq, nkv, hd = a.num_attention_heads, a.num_key_value_heads, a.head_dim
+        sandwich = a.sandwich_norms
+        tap = list(tap or [])
+        h = self.embed_rows(ids.reshape(-1))
+        fused = torch.empty((L, len(tap) * H), dtype=torch.bfloat16, device=self.device) if tap else None
+        x = ops.rows_prep(h, norm_w=self.layers[0].in_norm, eps=eps, later=not sandwich)
+        for l, Lw in enumerate(self.layers):
+            slots = [i for i, t in enumerate(tap) if t == l]
+            copy = fused[:, slots[0] * H:(slots[0] + 1) * H] if slots else None
+            last = l == a.num_hidden_layers - 1
+            next_norm = None if last else self.layers[l + 1].in_norm
+            k_pool, v_pool, k_sb, v_sb = cache.layer_args(l)
+            inv_freq = self.inv_freq_local if a.is_sliding(l) else self.inv_freq
+            q = ops.qkv_rope_append(ops.w8_rows(x, Lw.qkv), 1, L, nq, nkv, hd, Lw.q_norm, Lw.k_norm, eps, inv_freq,
+                                    cache.seq_lens, cache.block_table, cache.page, cache.kv_dtype, k_pool, v_pool,
+                                    k_sb, v_sb)
+            o = ops.attention_rows(q, 1, L, nq, nkv, hd, a.attn_scale, cache.seq_lens, cache.max_ctx,
+                                   cache.block_table, cache.page, cache.kv_dtype, k_pool, v_pool, k_sb, v_sb,
+                                   causal=True, window=a.window(l))
+            o = ops.rows_prep(o)
+            if sandwich:
+                y = ops.w8_rows(o, Lw.o)
+                x = ops.rows_prep(h, part=y, part_norm_w=Lw.attn_out_norm, norm_w=Lw.post_norm, eps=eps)
+            else:
+                ops.w8_rows(o, Lw.o, epi=ops.DSK_EPI_RESIDUAL, h=h)
+                x = ops.rows_prep(h, norm_w=Lw.post_norm, eps=eps, later=True)
+            act = ops.rows_prep(ops.w8_rows(x, Lw.gate_up, epi=self.act_epi))
+            if sandwich:
+                y = ops.w8_rows(act, Lw.down)
+                x = ops.rows_prep(h, part=y, part_norm_w=Lw.ff_out_norm, norm_w=next_norm, eps=eps, copy=copy,
+                                  out=not last)
+            else:
+                ops.w8_rows(act, Lw.down, epi=ops.DSK_EPI_RESIDUAL, h=h, copy=copy)
+                x = None if last else ops.rows_prep(h, norm_w=next_norm, eps=eps, later=True)
+            for extra in slots[1:]:
+                fused[:, extra * H:(extra + 1) * H].copy_(copy)
+        out = None
+        if logits != "none":
+            pack = ops.pack(h[-1:], self.norm, eps) if sandwich else ops.pack_rn(M=1, K=H, h=h[-1:], norm_w=self.norm,
+                                                                                 eps=eps)
+            out = torch.empty((1, a.vocab_size), dtype=torch.float32, device=self.device)
+            ops.w8_gemm(pack, self.lm_head, out=out, softcap=a.final_logit_softcapping or 0.0)
+            out = out.view(1, 1, -1)
+        ops.lens_add(cache.seq_lens, None, L)
+        cache.note_lengths([n + L for n in cache.lengths])
+        return out, (fused.view(1, L, -1) if fused is not None else None)
 
     # ------------------------------------------------------------------ dense prefill
     def keep_dense_weights(self, keep: bool = True) -> int:

@@ -1,0 +1,171 @@
+"""GPU: the products of many rows (dsk_rows_prep, dsk_w8_rows) at the edges of every tile the planner
+picks, and the many-row attention (dsk_attention_rows) at head_dim 128 and 256, against float64.
+
+A product's error: each of its two sums (scaled code products, bias products) accumulates at most K
+float32 terms, so K * 2^-24 of the sum of magnitudes, and the store rounds to bf16 (2^-8 of the
+value, 2^-9 for the rounding and as much for a flip of the input's own rounding in the reference)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): the plan each reaches (64-row blocks x column tiles, groups per step, K slices)
+SHAPES = [
+    (1, 48, 256),        # 1 x 1: an odd number of column tiles
+    (65, 32, 256),       # 1 x 2, two slices (four groups), a second block of one row
+    (70, 256, 512),      # 1 x 2, four slices
+    (190, 4096, 256),    # 1 x 4, four slices
+    (129, 4160, 512),    # 2 x 4, four slices
+    (130, 8192, 768),    # 2 x 4, two slices
+    (515, 16384, 256),   # 2 x 4, one slice (a 256-row tile would pad too much)
+    (1024, 8192, 256),   # 4 x 4
+    (203, 256, 8192 + 256),  # more groups than one step of the bias term
+]
+
+
+def _weight(N, K, bits, paired, dev):
+    from mlx_dspark.ops import W8Weight
+    g = torch.Generator(device=dev).manual_seed(N + K + bits)
+    q, s, b = W8Weight.quantize_mlx(torch.randn(N, K, generator=g, device=dev) * 0.02, bits)
+    qs = q.double().view(N, K // 64, 64) * s.double()[..., None]
+    bb = b.double()[..., None].expand(N, K // 64, 64)
+    return W8Weight.from_mlx(q, s, b, paired, bits), (qs + bb).reshape(N, K), (qs + bb.abs()).reshape(N, K)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("bits", [8, 4])
+def test_products_of_many_rows(dev, M, N, K, bits):
+    from mlx_dspark.ops import DSK_EPI_GEGLU, DSK_EPI_RESIDUAL, DSK_EPI_SWIGLU, rows_prep, w8_rows
+    print(f"rows M={M} N={N} K={K} bits={bits}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + bits)
+    wide = (torch.randn(M, K + 64, generator=g, device=dev) * 3).to(torch.bfloat16)
+    h = wide[:, :K]                                       # strided rows
+    norm = (1 + 0.2 * torch.randn(K, generator=g, device=dev)).to(torch.bfloat16)
+    eps = 1e-6
+    W, w64, mag = _weight(N, K, bits, False, dev)
+    x64 = (h.float() * norm.float()).to(torch.bfloat16).double()
+    r = torch.rsqrt(h.double().square().mean(1, keepdim=True) + eps)
+    ref, bound = (x64 @ w64.T) * r, K * 2.0 ** -24 * (x64.abs() @ mag.T) * r
+    x = rows_prep(h, norm_w=norm, eps=eps, later=True)
+    y = w8_rows(x, W)
+    assert bool(((y.double() - ref).abs() <= bound + ref.abs() * 2.0 ** -8).all())
+    # residual add, with a strided copy
+    res = torch.randn(M, N, generator=g, device=dev).to(torch.bfloat16)
+    hh, taps = res.clone(), torch.zeros((M, 2 * N), dtype=torch.bfloat16, device=dev)
+    w8_rows(x, W, epi=DSK_EPI_RESIDUAL, h=hh, copy=taps[:, N:])
+    want = res.double() + ref
+    assert bool(((hh.double() - want).abs() <= bound + want.abs() * 2.0 ** -8).all())
+    assert torch.equal(taps[:, N:], hh) and not bool(taps[:, :N].any())
+    if N % 32:
+        return
+    Wp, w64, mag = _weight(N, K, bits, True, dev)
+    ref = (x64 @ w64.T) * r
+    gate, up = ref[:, :N // 2], ref[:, N // 2:]
+    for epi, act in ((DSK_EPI_SWIGLU, torch.nn.functional.silu(gate)),
+                     (DSK_EPI_GEGLU, torch.nn.functional.gelu(gate, approximate="tanh"))):
+        y, want = w8_rows(x, Wp, epi=epi), act * up
+        # three bf16 roundings (gate, up, act) of factors of at most slope 1.13, and the store's
+        err = (y.double() - want).abs() - 2.0 ** -6 * ((gate.abs() + act.abs()) * up.abs())
+        assert float(err.max()) <= float(bound.max()) * float(ref.abs().max()) * 4
+
+
+@pytest.mark.parametrize("M,K", [(1, 64), (3, 4096), (67, 4160), (130, 12288), (5, 24576)])
+def test_prepared_rows(dev, M, K):
+    """The residual add and norms against float64, the operand order, and the group sums' terms."""
+    from mlx_dspark.ops import rows_prep
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    rnd = lambda: (torch.randn(M, K, generator=g, device=dev) * 2).to(torch.bfloat16)
+    w1, w2 = ((1 + 0.3 * torch.randn(K, generator=g, device=dev)).to(torch.bfloat16) for _ in range(2))
+    h, y, copy, eps = rnd(), rnd(), torch.zeros((M, K), dtype=torch.bfloat16, device=dev), 1e-6
+    h0 = h.clone()
+    x = rows_prep(h, part=y, part_norm_w=w1, copy=copy, norm_w=w2, eps=eps)
+    rms = lambda t: t * torch.rsqrt(t.square().mean(1, keepdim=True) + eps)
+    h64 = h0.double() + rms(y.double()) * w1.double()
+    assert bool(((h.double() - h64).abs() <= 2.0 ** -7 * (h64.abs() + rms(y.double()).abs() * w1.double().abs())).all())
+    assert torch.equal(h, copy)
+    Mp, G = (M + 15) // 16 * 16, K // 64
+    rows = x.data.view(Mp // 16, G, 2, 4, 16, 8).permute(0, 4, 1, 3, 2, 5).reshape(Mp, K)[:M]
+    x64 = rms(h.double()) * w2.double()
+    assert bool(((rows.double() - x64).abs() <= x64.abs() * 2.0 ** -7 + 1e-6).all())
+    Gp = (G + 63) // 64 * 64
+    xt = x.xt.view(3, Mp // 16, Gp // 64, 2, 4, 16, 8).permute(0, 1, 5, 2, 4, 3, 6).reshape(3, Mp, Gp)[:, :M]
+    sums = rows.double().view(M, G, 64).sum(2)
+    mags = rows.double().abs().view(M, G, 64).sum(2)
+    assert bool(((xt.double().sum(0)[:, :G] - sums).abs() <= mags * 2.0 ** -20).all())
+    assert not bool(xt[:, :, G:].any())
+    # without a norm the operand is the rows themselves
+    plain = rows_prep(h)
+    assert torch.equal(plain.data.view(Mp // 16, G, 2, 4, 16, 8).permute(0, 4, 1, 3, 2, 5).reshape(Mp, K)[:M], h)
+
+
+@pytest.mark.parametrize("hd,kv_bits,lens,W,nq,nkv,causal,window", [
+    (128, 8, [0], 203, 8, 2, True, 0),            # 64-row blocks
+    (128, None, [5, 700], 1100, 64, 2, True, 0),  # 256-row blocks (G = 32)
+    (128, None, [70], 65, 2, 2, True, 33),
+    (256, None, [0], 1027, 4, 2, True, 0),
+    (256, 8, [900, 3], 65, 8, 8, True, 130),      # windows that start inside a block
+    (256, None, [40], 129, 4, 1, False, 0),
+])
+def test_many_row_attention(dev, hd, kv_bits, lens, W, nq, nkv, causal, window):
+    """Against a float64 softmax over the stored keys: probabilities within 2^-26 and float32 sums
+    leave the output's own bf16 rounding (2^-9) and the queries' and keys' products (float32) well
+    inside 2^-7 of the largest output."""
+    from mlx_dspark import ops
+    from mlx_dspark.kv import PagedKVCache
+    print(f"attention rows hd={hd} kv_bits={kv_bits} lens={lens} W={W} window={window}", flush=True)
+    B = len(lens)
+    cache = PagedKVCache(1, B, nkv, hd, max(lens) + W + 64, kv_bits=kv_bits, spare_pages=3)
+    g = torch.Generator(device=dev).manual_seed(sum(lens) + W + hd)
+    perm = torch.randperm(cache.n_pages, generator=torch.Generator().manual_seed(W))[: B * cache.max_pages]
+    cache.block_table.copy_(perm.view(B, cache.max_pages).to(torch.int32))
+    pools = []
+    for pool, sb in ((cache.k[0], cache.k_sb[0]), (cache.v[0], cache.v_sb[0])):
+        if kv_bits is None:
+            pool.copy_(torch.randn(pool.shape, generator=g, device=dev))
+            pools.append(pool.double())
+            continue
+        pool.copy_(torch.randint(0, 256, pool.shape, generator=g, device=dev))
+        sc = (0.01 + 0.01 * torch.rand(sb.shape, generator=g, device=dev)).to(torch.bfloat16)
+        bi = (-2.0 + torch.rand(sb.shape, generator=g, device=dev)).to(torch.bfloat16)
+        sb.copy_((sc.view(torch.int16).int() & 0xFFFF) | (bi.view(torch.int16).int() << 16))
+        v = pool.float().view(*pool.shape[:-1], hd // 64, 64) * sc.float()[..., None] + bi.float()[..., None]
+        pools.append(v.view(pool.shape).to(torch.bfloat16).double())
+    cache.set_lengths(lens)
+    q = torch.randn(B * W, nq * hd, generator=g, device=dev).to(torch.bfloat16)
+    out = ops.attention_rows(q, B, W, nq, nkv, hd, hd ** -0.5, cache.seq_lens, cache.max_ctx, cache.block_table,
+                             cache.page, cache.kv_dtype, *cache.layer_args(0), causal=causal, window=window)
+    got = out.double().view(B, W, nq, hd)
+    for b, L0 in enumerate(lens):
+        n = L0 + W
+        K, V = (p[cache.block_table[b].long()].transpose(1, 2).reshape(-1, nkv, hd)[:n] for p in pools)
+        pos = torch.arange(L0, n, device=dev)[:, None]
+        j = torch.arange(n, device=dev)[None, :]
+        ok = j <= pos if causal else torch.ones((W, n), dtype=torch.bool, device=dev)
+        if window:
+            ok = ok & (j > pos - window)
+        for t in range(nq):
+            sc = (q.double().view(B, W, nq, hd)[b, :, t] @ K[:, t * nkv // nq].T) * hd ** -0.5
+            ref = torch.softmax(sc.masked_fill(~ok, -float("inf")), -1) @ V[:, t * nkv // nq]
+            assert float((got[b, :, t] - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())
+
+
+def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
+    """A Gemma-style prompt of one piece and a few rows more: the same cache, taps and logits as
+    64-row forward passes, up to the rounding flips of other sums (2e-2 of the largest value)."""
+    from mlx_dspark import synthetic
+    from mlx_dspark.qwen3 import PREFILL_CHUNK
+    model = synthetic.build_target("tiny-gemma", seed=41)
+    n = PREFILL_CHUNK + 7
+    prompt = torch.randint(0, model.args.vocab_size, (n,), generator=torch.Generator().manual_seed(1)).tolist()
+    outs = []
+    for chunk in (64, 63):           # 63: forward passes
+        cache = model.make_cache(max_ctx=n + 64)
+        seen = []
+        logits, _ = model.prefill(prompt, cache, [0, 5], chunk=chunk, on_chunk=lambda f, pos: seen.append((pos, f)))
+        torch.cuda.synchronize()
+        assert cache.lengths[0] == n and int(cache.seq_lens[0]) == n
+        assert [p for p, _ in seen] == list(range(0, n, PREFILL_CHUNK if chunk == 64 else 63))
+        outs.append((logits, torch.cat([f for _, f in seen], dim=1), cache.k[5], cache.v[5]))
+    for a, b in zip(*outs):
+        assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
