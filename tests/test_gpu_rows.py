@@ -169,3 +169,60 @@ def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
         outs.append((logits, torch.cat([f for _, f in seen], dim=1), cache.k[5], cache.v[5]))
     for a, b in zip(*outs):
         assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
+
+
+@pytest.mark.parametrize("hd,nq,nkv,kv_bits,v_norm,B,W", [
+    (128, 4, 2, None, False, 1, 203), (128, 0, 3, 8, False, 2, 70), (128, 5, 1, 8, True, 1, 128),
+    (256, 4, 2, 8, False, 1, 131), (256, 2, 1, None, True, 3, 50), (512, 3, 1, 8, True, 1, 130),
+])
+def test_append_of_many_rows_equals_the_general_form(dev, hd, nq, nkv, kv_bits, v_norm, B, W):
+    """A workgroup per row (bf16 projections of 128 rows and more) against a wave per head, which the
+    same projection given as one f32 slice takes: only the order of the norm's float32 sums differs, so
+    a value may differ by one bf16 step (2^-7 of it) and a code by that step in units of its scale. Odd
+    head counts, rows past the block table (dropped) and uneven lengths."""
+    from mlx_dspark import ops
+    from mlx_dspark.kv import PagedKVCache
+    print(f"append hd={hd} nq={nq} nkv={nkv} kv_bits={kv_bits} v_norm={v_norm} B={B} W={W}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(hd + W)
+    M, N = B * W, (nq + 2 * nkv) * hd
+    qkv = (torch.randn(M, N, generator=g, device=dev) * 2).to(torch.bfloat16)
+    gains = [(1 + 0.2 * torch.randn(hd, generator=g, device=dev)).to(torch.bfloat16) for _ in range(3)]
+    inv = ops.rope_inv_freq(hd, 1e6, dev)
+    outs = []
+    for x in (qkv, qkv.float()[None]):
+        cache = PagedKVCache(1, B, nkv, hd, 192, kv_bits=kv_bits)
+        cache.set_lengths([(37 * b + 5) % 100 for b in range(B)])
+        q = ops.qkv_rope_append(x.contiguous(), B, W, nq, nkv, hd, gains[0], gains[1], 1e-6, inv, cache.seq_lens,
+                                cache.block_table, cache.page, cache.kv_dtype, *cache.layer_args(0),
+                                v_norm=gains[2] if v_norm else None)
+        kv = []
+        for pool, sb in ((cache.k[0], cache.k_sb[0]), (cache.v[0], cache.v_sb[0])):
+            if kv_bits:
+                s, b = ((sb << 16).view(torch.float32)[..., None], (sb & -65536).view(torch.float32)[..., None])
+                kv.append((pool.float().view(*sb.shape, 64) * s + b).view(pool.shape))
+                kv.append(s.expand(*sb.shape, 64).reshape(pool.shape))
+            else:
+                kv += [pool.float(), torch.zeros_like(pool, dtype=torch.float32)]
+        outs.append((q, kv))
+    (qa, ka), (qb, kb) = outs
+    if nq:
+        assert bool(((qa.float() - qb.float()).abs() <= 2.0 ** -7 * qb.float().abs() + 2.0 ** -7).all())
+        assert float((qa != qb).float().mean()) < 0.01
+    for i in (0, 2):
+        step = ka[i + 1].abs() + 2.0 ** -7 * kb[i].abs().amax(-1, keepdim=True)
+        assert bool(((ka[i] - kb[i]).abs() <= step).all())
+        assert float((ka[i] != kb[i]).float().mean()) < 0.02
+
+
+@pytest.mark.parametrize("n,H", [(1, 64), (3, 1024), (130, 4096)])
+def test_embed_in_whole_pieces_equals_the_general_form(dev, n, H):
+    """16 codes per thread (aligned rows and outputs) against one element per thread (an output row
+    stride that is no multiple of 8), bit for bit, with ids out of range."""
+    from mlx_dspark.ops import W8Table, W8Weight, w8_embed
+    g = torch.Generator(device=dev).manual_seed(n + H)
+    t = W8Table(*W8Weight.quantize_mlx(torch.randn(50, H, generator=g, device=dev)))
+    ids = torch.randint(0, 50, (n,), generator=g, device=dev, dtype=torch.int32)
+    ids[-1] = 77
+    odd = torch.zeros((n, H + 3), dtype=torch.bfloat16, device=dev)[:, :H]
+    for scale in (1.0, 62.0):
+        assert torch.equal(w8_embed(ids, t, scale), w8_embed(ids, t, scale, out=odd))
