@@ -54,7 +54,11 @@ struct PrepArgs {
 template <int NV>
 __global__ __launch_bounds__(kPrepThreads) void rows_prep_kernel(PrepArgs a) {
   __shared__ float red[kPrepThreads / 64];
-  const int64_t m = blockIdx.x;
+  // the 16 rows of a tile go to one XCD (workgroups go round robin to the eight): their 16-byte pieces
+  // of the operand order share cache lines, which that XCD's L2 then writes whole (2048 rows of 20480:
+  // 87 -> 52 us; 1027 of 15360: 34 -> 17.5)
+  const int64_t m = (((int64_t)blockIdx.x / 128) * 8 + blockIdx.x % 8) * 16 + (blockIdx.x / 8) % 16;
+  if (m >= a.M) return;
   const int tid = threadIdx.x;
   const int64_t nchunk = a.K / 8;
   u32x4 hv[NV], yv[NV], yw[NV], wv[NV];
@@ -512,7 +516,7 @@ extern "C" int dsk_rows_prep(uint16_t* h, int64_t ldh, const uint16_t* y, int64_
   const int64_t G = K / 64;
   PrepArgs a{h, ldh, y, ldy, y_norm_w, copy, ldc, K, G, (G + 63) / 64 * 64, M, norm_w, later, eps, x, xt,
              (int64_t)((M + 15) / 16 * 16) * ((G + 63) / 64 * 64), rsc};
-  const dim3 grid((unsigned)M), blk(kPrepThreads);
+  const dim3 grid((unsigned)(ceil_div(M, 128) * 128)), blk(kPrepThreads);
   const hipStream_t st = as_stream(stream);
   switch (ceil_div(K / 8, kPrepThreads)) {
     case 1: hipLaunchKernelGGL(rows_prep_kernel<1>, grid, blk, 0, st, a); break;
