@@ -1405,6 +1405,14 @@ constexpr int kPfMaxPages = 1024;             // page ids of a row block's keys 
 // with 4 waves and this bound, 239 us with 8 waves sharing each block's dequantisation (one bf16 term
 // of P). 4 waves of one tile where the 256-row blocks leave CUs idle, and at head_dim 256, where the
 // two K/V buffers fill the LDS.
+// a loaded chunk as four words of two bf16 values
+template <int KVT>
+__device__ __forceinline__ u32x4 chunk_words(const Chunk8& c) {
+  uint16_t h[8];
+  chunk_bf16<KVT>(c, h);
+  return *reinterpret_cast<const u32x4*>(h);
+}
+
 template <int HD, int KVT, int TERMS, int NW, int TPW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, 2))) void attention_prefill_kernel(AttnArgs a) {
   constexpr int KS = HD / 32, DT = HD / 16, NKT = kPfKeys / 16, NTHR = NW * 64;
@@ -1416,7 +1424,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
   __shared__ __attribute__((aligned(16))) uint16_t ks[2][kPfKeys * kPfKRow];
   __shared__ __attribute__((aligned(16))) uint32_t vt[2][HD * kPfVRow / 2];
   __shared__ int pgs[kPfMaxPages];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __shared__ int toks[4][kPfKeys];  // pool tokens of the keys of blocks n .. n + 3
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int bk = blockIdx.x, b = bk / a.nkv, kvh = bk % a.nkv;
   const int nrb = (a.R + kPfRows - 1) / kPfRows;
   const int rb = nrb - 1 - (int)blockIdx.y;
@@ -1455,23 +1464,29 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();  // the page ids
 
-  auto tok_of = [&](int j) -> int64_t {
-    j = min(j, j_end - 1);  // keys past the range load the last one and are zeroed in LDS
-    return ((int64_t)pgs[j / a.page - pg0] * a.nkv + kvh) * a.page + (j % a.page);
+  // pool token of key t of block n (keys past the range: the last one, zeroed in LDS). Found once per
+  // key, a block ahead of its loads: the division by the page size costs ~20 instructions, and every
+  // thread loads pieces of 4 (head_dim 128) to 24 (256) keys per block
+  auto find_token = [&](int n, int t) {
+    const int j = min(j_beg + n * kPfKeys + t, j_end - 1);
+    toks[n & 3][t] = (pgs[j / a.page - pg0] * a.nkv + kvh) * a.page + j % a.page;
   };
+  if (nb > 0 && threadIdx.x < 3 * kPfKeys) find_token(threadIdx.x / kPfKeys, threadIdx.x % kPfKeys);
+  __syncthreads();
   Chunk8 kc[CK], vc[CV][2];
-  auto issue = [&](int j0) {
+  auto issue = [&](int n) {
+    const int* tk = toks[n & 3];
 #pragma unroll
     for (int ci = 0; ci < CK; ++ci) {
       const int c = threadIdx.x + ci * NTHR;
-      load_chunk<KVT>(a.k_pool, a.k_sb, HD, tok_of(j0 + c / (HD / 8)), (c % (HD / 8)) * 8, kc[ci]);
+      load_chunk<KVT>(a.k_pool, a.k_sb, HD, tk[c / (HD / 8)], (c % (HD / 8)) * 8, kc[ci]);
     }
 #pragma unroll
     for (int ci = 0; ci < CV; ++ci) {
       const int c = threadIdx.x + ci * NTHR;
       const int kp = c % (kPfKeys / 2), d0 = (c / (kPfKeys / 2)) * 8;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) load_chunk<KVT>(a.v_pool, a.v_sb, HD, tok_of(j0 + 2 * kp + u), d0, vc[ci][u]);
+      for (int u = 0; u < 2; ++u) load_chunk<KVT>(a.v_pool, a.v_sb, HD, tk[2 * kp + u], d0, vc[ci][u]);
     }
   };
   // the loaded words stay opaque until to_lds: the compiler would otherwise unpack the 8-bit
@@ -1493,9 +1508,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     for (int ci = 0; ci < CK; ++ci) {
       const int c = threadIdx.x + ci * NTHR;
       const int key = c / (HD / 8), d0 = (c % (HD / 8)) * 8;
-      uint16_t h[8];
-      chunk_bf16<KVT>(kc[ci], h);
-      u32x4 w = *reinterpret_cast<const u32x4*>(h);
+      u32x4 w = chunk_words<KVT>(kc[ci]);
       if (j_lo + key >= j_hi) w = u32x4{0, 0, 0, 0};
       *reinterpret_cast<u32x4*>(&ks[buf][key * kPfKRow + d0]) = w;
     }
@@ -1503,14 +1516,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     for (int ci = 0; ci < CV; ++ci) {
       const int c = threadIdx.x + ci * NTHR;
       const int kp = c % (kPfKeys / 2), d0 = (c / (kPfKeys / 2)) * 8;
-      const int j0 = j_lo + 2 * kp;
-      uint16_t h0[8], h1[8];
-      chunk_bf16<KVT>(vc[ci][0], h0);
-      chunk_bf16<KVT>(vc[ci][1], h1);
-      const bool z0 = j0 >= j_hi, z1 = j0 + 1 >= j_hi;
+      u32x4 w0 = chunk_words<KVT>(vc[ci][0]), w1 = chunk_words<KVT>(vc[ci][1]);
+      if (j_lo + 2 * kp >= j_hi) w0 = u32x4{0, 0, 0, 0};
+      if (j_lo + 2 * kp + 1 >= j_hi) w1 = u32x4{0, 0, 0, 0};
+      uint32_t* dst = &vt[buf][(d0 * kPfVRow) / 2 + kp];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        vt[buf][((d0 + e) * kPfVRow) / 2 + kp] = (uint32_t)(z0 ? 0 : h0[e]) | ((uint32_t)(z1 ? 0 : h1[e]) << 16);
+      for (int e = 0; e < 4; ++e) {  // dims d0 + 2 e, d0 + 2 e + 1 of both keys
+        dst[(2 * e) * kPfVRow / 2] = __builtin_amdgcn_perm(w1[e], w0[e], 0x05040100u);
+        dst[(2 * e + 1) * kPfVRow / 2] = __builtin_amdgcn_perm(w1[e], w0[e], 0x07060302u);
+      }
     }
   };
 
@@ -1635,9 +1649,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
   };
 
   if (nb > 0) {
-    issue(j_beg);
+    issue(0);
     to_lds(0, j_beg, min(j_end, j_beg + kPfKeys));
-    if (nb > 1) issue(j_beg + kPfKeys);
+    if (nb > 1) issue(1);
   }
   __syncthreads();
 #pragma unroll 1
@@ -1646,13 +1660,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     // a wave whose rows see none of the block skips it (causal: all its rows before the block;
     // window: all its rows' windows past it)
     const bool skip = !wave_live || (causal && j_lo > wq_hi) || (causal && window > 0 && j_hi - 1 < wq_lo - window + 1);
-    if (!skip) compute(n & 1, j_lo, j_hi);
+    // of eight waves, half stage the next block first: the waves of a SIMD then are in different phases
+    // (the 4096-token layer 275 -> 268 us)
+    const bool stage_first = NW == 8 && wv >= NW / 2;
+    if (!skip && !stage_first) compute(n & 1, j_lo, j_hi);
     if (n + 1 < nb) {
       // the other buffer was last read in block n - 1, which every wave finished before the
       // previous barrier
       to_lds((n + 1) & 1, j_lo + kPfKeys, min(j_end, j_lo + 2 * kPfKeys));
-      if (n + 2 < nb) issue(j_lo + 2 * kPfKeys);
+      if (n + 2 < nb) issue(n + 2);
+      // slot (n - 1) & 3, whose block was loaded two barriers ago
+      if (n + 3 < nb && threadIdx.x < kPfKeys) find_token(n + 3, threadIdx.x);
     }
+    if (!skip && stage_first) compute(n & 1, j_lo, j_hi);
     __syncthreads();
   }
 
