@@ -1403,7 +1403,8 @@ constexpr int kPfMaxPages = 1024;             // page ids of a row block's keys 
 // Shapes: 8 waves of two tiles at head_dim 128 (256 rows; at most 256 VGPRs, two waves per SIMD, whose
 // staging and MFMAs interleave). On the 4096-token Qwen3-8B layer: 436 us with 4 waves and no bound, 299 us
 // with 4 waves and this bound, 239 us with 8 waves sharing each block's dequantisation (one bf16 term
-// of P). 4 waves of one tile where the 256-row blocks leave CUs idle, and at head_dim 256, where the
+// of P); with two terms of P 326 us, 263 us (522 TFLOP/s) since the tokens are found once per key and
+// half the waves stage first. 4 waves of one tile where the 256-row blocks leave CUs idle, and at head_dim 256, where the
 // two K/V buffers fill the LDS.
 // a loaded chunk as four words of two bf16 values
 template <int KVT>
