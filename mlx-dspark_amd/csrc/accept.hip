@@ -291,7 +291,8 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(int64_t V, const float
 // ============================================================================= sampled paths
 constexpr int kST = 512;              // threads per workgroup
 constexpr int kSW = kST / 64;
-constexpr int kMaxSlices = 32;        // workgroups per row in the row passes
+constexpr int kFewRows = 4;           // rows up to which a workgroup per CU holds every slice at kMaxSlices
+constexpr int kMaxSlices = 64;        // workgroups per row in the row passes (a lane each in row_max)
 constexpr int kEPT = 32;              // elements per thread in the gather pass: slice <= 16384
 constexpr int kMaxDrawSlices = 128;   // workgroups per draw in the draw passes (<= kST)
 constexpr int kDrawEPT = 8;           // elements per thread in the draw pass: draw slice <= 4096
@@ -383,7 +384,10 @@ __device__ __forceinline__ float yv(float x, int mul, float T, float inv_t) {
 }
 __device__ __forceinline__ uint32_t samp_offset(const SampArgs& a) { return a.offset_dev ? a.offset_dev[0] : a.offset; }
 
+// the row's max from its slices', a lane per slice: every lane of the calling wave takes part (one
+// round trip); few slices are read in turn
 __device__ __forceinline__ float row_max(const SampArgs& a, int r) {
+  if (a.S > 16) return wave_max(a.gmax[r * kMaxSlices + min((int)(threadIdx.x & 63), a.S - 1)]);
   float m = a.gmax[r * kMaxSlices];
   for (int s = 1; s < a.S; ++s) m = fmaxf(m, a.gmax[r * kMaxSlices + s]);
   return m;
@@ -583,60 +587,77 @@ __device__ inline void bucket_window(uint32_t b, float& lo, float& hi) {
 // ---- pass 3a (truncation), one workgroup per row: the threshold buckets from the merged
 // histogram (buckets scanned in descending order, thread t holding bucket kL1 - 1 - t), the
 // mass and count above them, and the window of x = y - m the gather stages.
-__global__ __launch_bounds__(kST) void samp_select_kernel(SampArgs a) {
-  __shared__ uint64_t sh[kSW];
-  __shared__ uint32_t sel[4];
-  __shared__ uint64_t selw[2];
-  const int r = blockIdx.x;
+struct SelSmem {
+  uint64_t sh[kSW];
+  uint64_t selw[2];
+  uint32_t sel[4];
+  RowInfo info;
+};
+
+// every thread of the workgroup returns the row's RowInfo. With at most kFewRows rows the gather's
+// workgroups each do this for themselves (one chained sampled draw, one row of 151936: select 4.2 +
+// gather 8.0 us in two launches, 9.8 in one; the whole chain of seven draws 343 -> 313 us, together
+// with 64 slices instead of 32). With 12 rows at 64 slices the smaller slices' fixed costs (histogram
+// merge, clears) lost 20 %, and with 132 rows the repeated selection 3 %: those keep the two launches.
+__device__ RowInfo select_row(const SampArgs& a, int r, SelSmem& sm) {
   const uint64_t Z = a.zsum[r];
-  const uint64_t TP = a.do_p ? top_p_target(a.top_p, Z) : 0;
   const int bb = kL1 - 1 - (int)threadIdx.x;
   const uint64_t c = a.hcnt[r * kL1 + bb];
   const uint64_t w = a.hwgt[r * kL1 + bb];
+  const float m = row_max(a, r);
+  const uint64_t TP = a.do_p ? top_p_target(a.top_p, Z) : 0;
   if (threadIdx.x == 0) {
-    sel[0] = kNone;
-    sel[1] = kNone;
+    sm.sel[0] = kNone;
+    sm.sel[1] = kNone;
   }
   uint64_t tot;
-  const uint64_t ic = block_scan512(c, sh, tot);
-  const uint64_t iw = block_scan512(w, sh, tot);
+  const uint64_t ic = block_scan512(c, sm.sh, tot);
+  const uint64_t iw = block_scan512(w, sm.sh, tot);
   if (a.do_k && ic - c < (uint64_t)a.top_k && ic >= (uint64_t)a.top_k) {
-    sel[0] = (uint32_t)bb;
-    sel[2] = (uint32_t)(ic - c);
-    selw[0] = iw - w;
+    sm.sel[0] = (uint32_t)bb;
+    sm.sel[2] = (uint32_t)(ic - c);
+    sm.selw[0] = iw - w;
   }
   if (a.do_p && TP > 0 && iw - w < TP && iw >= TP) {
-    sel[1] = (uint32_t)bb;
-    selw[1] = iw - w;
+    sm.sel[1] = (uint32_t)bb;
+    sm.selw[1] = iw - w;
   }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  RowInfo inf;
-  inf.bk = sel[0];
-  inf.bp = sel[1];
-  inf.above_k = inf.bk == kNone ? 0 : sel[2];
-  inf.pad = 0;
-  inf.wabove_k = inf.bk == kNone ? 0 : selw[0];
-  inf.wabove_p = inf.bp == kNone ? 0 : selw[1];
-  inf.tp = TP;
-  const uint32_t bq = (inf.bp == inf.bk) ? kNone : inf.bp;
-  float klo, khi, qlo, qhi;
-  bucket_window(inf.bk, klo, khi);
-  bucket_window(bq, qlo, qhi);
-  inf.wlo = fminf(klo, qlo);
-  inf.whi = fmaxf(khi, qhi);
-  // with T == 1 the window moves to the raw values (y = v): v - m in [wlo, whi] holds for every
-  // v in [m + wlo, m + whi] widened by one part in 2^20 of the bounds' magnitudes
-  const float m = row_max(a, r);
-  inf.vlo = (m + inf.wlo) - fabsf(m + inf.wlo) * 0x1p-20f - 0x1p-100f;
-  inf.vhi = (m + inf.whi) + fabsf(m + inf.whi) * 0x1p-20f + 0x1p-100f;
-  a.info[r] = inf;
+  if (threadIdx.x == 0) {
+    RowInfo inf;
+    inf.bk = sm.sel[0];
+    inf.bp = sm.sel[1];
+    inf.above_k = inf.bk == kNone ? 0 : sm.sel[2];
+    inf.pad = 0;
+    inf.wabove_k = inf.bk == kNone ? 0 : sm.selw[0];
+    inf.wabove_p = inf.bp == kNone ? 0 : sm.selw[1];
+    inf.tp = TP;
+    const uint32_t bq = (inf.bp == inf.bk) ? kNone : inf.bp;
+    float klo, khi, qlo, qhi;
+    bucket_window(inf.bk, klo, khi);
+    bucket_window(bq, qlo, qhi);
+    inf.wlo = fminf(klo, qlo);
+    inf.whi = fmaxf(khi, qhi);
+    // with T == 1 the window moves to the raw values (y = v): v - m in [wlo, whi] holds for every
+    // v in [m + wlo, m + whi] widened by one part in 2^20 of the bounds' magnitudes
+    inf.vlo = (m + inf.wlo) - fabsf(m + inf.wlo) * 0x1p-20f - 0x1p-100f;
+    inf.vhi = (m + inf.whi) + fabsf(m + inf.whi) * 0x1p-20f + 0x1p-100f;
+    sm.info = inf;
+  }
+  __syncthreads();
+  return sm.info;
+}
+
+__global__ __launch_bounds__(kST) void samp_select_kernel(SampArgs a) {
+  __shared__ SelSmem sm;
+  const RowInfo inf = select_row(a, blockIdx.x, sm);
+  if (threadIdx.x == 0) a.info[blockIdx.x] = inf;
 }
 
 // ---- pass 3b (truncation): the candidates of the threshold buckets. A cheap window test
 // stages each wave's window elements in LDS by ballot; the exact keys of the staged elements are
 // then computed densely, so exp never runs divergently.
-template <bool VEC, bool TONE>
+template <bool VEC, bool TONE, bool SEL>
 __global__ __launch_bounds__(kST) void samp_gather_kernel(SampArgs a) {
   __shared__ uint64_t sh[kSW];
   __shared__ uint32_t base[2];
@@ -649,7 +670,14 @@ __global__ __launch_bounds__(kST) void samp_gather_kernel(SampArgs a) {
   const int n = (int)(hi - lo);
   SliceRegs<VEC> xr;
   xr.load(x, lo, hi);
-  const RowInfo inf = a.info[r];
+  RowInfo inf;
+  if constexpr (SEL) {  // few rows: every workgroup selects for itself, one launch less
+    __shared__ SelSmem sm;
+    inf = select_row(a, r, sm);
+    if (s == 0 && threadIdx.x == 0) a.info[r] = inf;
+  } else {
+    inf = a.info[r];
+  }
   const float m = row_max(a, r);
   const uint32_t bk = inf.bk, bq = (inf.bp == inf.bk) ? kNone : inf.bp;
   if (bk == kNone && bq == kNone) return;
@@ -1087,12 +1115,12 @@ __host__ inline void samp_bind(SampArgs& a, void* base, const SampLayout& L) {
 }
 
 // slices per row: at least enough for the gather pass's registers, about 1024 workgroups in
-// all, at most kMaxSlices, never slices shorter than 512 elements
+// all, at most kMaxSlices (half of it beyond kFewRows), never slices shorter than 512 elements
 __host__ inline int samp_slices(int rows, int64_t V) {
   int64_t S = ceil_div(1024, rows);
   S = std::min<int64_t>(S, std::max<int64_t>(1, V / 512));
   S = std::max<int64_t>(S, ceil_div(V, kMaxSlice));
-  return (int)std::min<int64_t>(S, kMaxSlices);
+  return (int)std::min<int64_t>(S, rows <= kFewRows ? kMaxSlices : kMaxSlices / 2);
 }
 
 __host__ inline int64_t samp_slice_len(int64_t V, int S) { return (ceil_div(V, S) + 3) & ~(int64_t)3; }
@@ -1130,12 +1158,17 @@ static int launch_sampled(SampArgs& a, int draws, hipStream_t st, const char* wh
   const dim3 blk(kST);
   const dim3 grow((unsigned)(rows * a.S));
   const bool one = a.T == 1.0f;
+  const bool few = rows <= kFewRows;
 #define DSK_ROW_PASSES(VEC_, ONE_)                                                 \
   hipLaunchKernelGGL((samp_max_kernel<VEC_, ONE_>), grow, blk, 0, st, a);          \
   hipLaunchKernelGGL((samp_stats_kernel<VEC_, ONE_>), grow, blk, 0, st, a);        \
   if (a.do_k || a.do_p) {                                                          \
-    hipLaunchKernelGGL(samp_select_kernel, dim3((unsigned)rows), blk, 0, st, a);   \
-    hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_>), grow, blk, 0, st, a);     \
+    if (few) {                                                                     \
+      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, true>), grow, blk, 0, st, a);  \
+    } else {                                                                       \
+      hipLaunchKernelGGL(samp_select_kernel, dim3((unsigned)rows), blk, 0, st, a); \
+      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, false>), grow, blk, 0, st, a); \
+    }                                                                              \
   }
   if (a.vec && one) {
     DSK_ROW_PASSES(true, true)
