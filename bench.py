@@ -168,7 +168,7 @@ def gemm_by_kernel(shapes: dict) -> list:
 def gemm_sweep(model, M: int, reps: int = 10) -> dict:
     """Plan sweep of the W8 GEMM at the verify-step shapes through the explicit-plan tuning
     entry (dsk_w8_gemm_rn_planned): every plan it accepts (slab tiles 1-8 dividing the tile
-    count, 1-, 2- or 4-group batches, 4 / 8 / 16 waves, 1-8 K splits for the partial sums, loads
+    count, 2- or 4-group batches, 4 / 8 / 16 waves, 1-8 K splits for the partial sums, loads
     pipelined or not), each timed as gemm_roofline times the planner's own (one launch per layer
     on that layer's weights in one graph, HIP events); the planner's choice is marked. The
     planner's rules (w8.hip, plan_gemm) were fitted to sweeps of this kind."""
@@ -204,7 +204,7 @@ def gemm_sweep(model, M: int, reps: int = 10) -> dict:
         for nt in (1, 2, 3, 4, 6, 8):
             if tiles % nt or (epi == SW and nt % 2):
                 continue
-            for u in (1, 2, 4):
+            for u in (2, 4):
                 for waves in (4, 8, 16):
                     for sk in ((1, 2, 3, 4, 5, 8) if epi == P else (1,)):
                         for pf in (0, 1):

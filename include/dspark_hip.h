@@ -160,7 +160,7 @@ int dsk_w8_gemm_rn(const uint16_t* x, const uint8_t* wt, const uint32_t* sb, int
 /* Tuning entry, with no counterpart in the reference: dsk_w8_gemm_rn with an explicit plan instead
  * of the library's own, for plan sweeps (the planner's rules were fitted from such sweeps):
  * slab_tiles 16-row weight tiles per workgroup (dividing N / 16; even for the gated epilogues),
- * batch_groups 1, 2 or 4 groups of 64 along K per load batch, waves 4 / 8 / 16, k_splits K splits
+ * batch_groups 2 or 4 groups of 64 along K per load batch, waves 4 / 8 / 16, k_splits K splits
  * (DSK_EPI_PARTIAL only: y then holds k_splits slices [M][N]), pipelined loads (1) or not (0).
  * A plan with no compiled kernel, or whose cross-wave reduction exceeds 64 KB of LDS, is
  * rejected with DSK_EINVAL. */

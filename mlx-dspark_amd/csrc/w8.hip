@@ -489,12 +489,8 @@ __device__ __forceinline__ void batch_compute(const Batch<MT, NT, U, BITS>& r, f
 // family is its own (smaller) kernel. PF: software-pipelined batch loads (two register sets).
 // EKR = EK + 4 * RS: RS, the row scale of a normed-later x, is compiled into its own kernels
 // (its registers would otherwise weigh on every plan).
-// Two waves per SIMD at least (256 registers): with more the compiler put the products into
-// accumulator registers of 4-wave plans and read every one back for its scaling (60 of 329 instructions
-// of a 3 x 4 batch).
 template <int MT, int NT, int U, int WAVES, int EKR, bool PF, int BITS>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVES <= 8 ? 2 : 4)))
-void w8_gemm_kernel(GemmArgs a) {
+__global__ __launch_bounds__(WAVES * 64) void w8_gemm_kernel(GemmArgs a) {
   constexpr int EK = EKR & 3;
   constexpr bool RS = EKR >= 4;
   const int lane = threadIdx.x & 63;
@@ -576,33 +572,21 @@ void w8_gemm_kernel(GemmArgs a) {
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __builtin_amdgcn_sched_barrier(0);
       }
-      // every load in the loop is unconditional (a load behind a bounds test made the compiler wait
-      // for all loads in flight at each batch), and the barriers keep each batch's loads ahead of the
-      // other batch's products; the last one or two batches follow the loop
-      int bt = wave;
-      for (; bt + 2 * WAVES < nbatch; bt += 2 * WAVES) {
-        batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)(bt + WAVES) * U, lane, rb);
-        __builtin_amdgcn_sched_barrier(0);
+      for (int bt = wave;;) {
+        if (bt + WAVES < nbatch) batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)(bt + WAVES) * U, lane, rb);
         batch_compute<MT, NT, U, BITS>(ra, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)(bt + 2 * WAVES) * U, lane, ra);
-        __builtin_amdgcn_sched_barrier(0);
+        bt += WAVES;
+        if (bt >= nbatch) break;
+        if (bt + WAVES < nbatch) batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)(bt + WAVES) * U, lane, ra);
         batch_compute<MT, NT, U, BITS>(rb, acc);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (bt + WAVES < nbatch) {
-        batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)(bt + WAVES) * U, lane, rb);
-        __builtin_amdgcn_sched_barrier(0);
-        batch_compute<MT, NT, U, BITS>(ra, acc);
-        batch_compute<MT, NT, U, BITS>(rb, acc);
-      } else {
-        batch_compute<MT, NT, U, BITS>(ra, acc);
+        bt += WAVES;
+        if (bt >= nbatch) break;
       }
     }
   } else {
-    // registers per thread: 512 / (waves per SIMD), at most 256; the batch, the accumulators, ~48 more
+    // registers per thread: 512 / (waves per SIMD); the batch, the accumulators and ~48 more
     constexpr bool kWholeBatch =
-        sizeof(Batch<MT, NT, U, BITS>) / 4 + MT * NT * 4 + 48 <= (WAVES <= 8 ? 256 : 2048 / WAVES);
+        sizeof(Batch<MT, NT, U, BITS>) / 4 + MT * NT * 4 + 48 <= 2048 / WAVES;
     for (int bt = wave; bt < nbatch; bt += WAVES) {
       Batch<MT, NT, U, BITS> r;
       batch_load<MT, NT, U, BITS>(a, t0, g_lo + (int64_t)bt * U, lane, r);
@@ -782,17 +766,21 @@ static const TunedPlan kTunedPlans[] = {
     {1, 4096, 12288, 3, 1, 2, 8, 1, false, 8},
     {1, 4096, 4096, 3, 1, 2, 16, 1, true, 8},
     {1, 24576, 4096, 1, 2, 2, 8, 1, false, 8},
-    // Qwen3-0.6B, 9-row verify: qkv 3.25 (3.60), gate_up 4.7 (6.37), head 38.5 (40.7)
+    // Qwen3-0.6B, 9-row verify: qkv 3.32 (3.60), gate_up 4.88 (6.37), head 38.8 (40.7)
     {1, 4096, 1024, 2, 1, 4, 4, 1, true, 8},
-    {1, 6144, 1024, 1, 2, 1, 16, 1, true, 8},
+    {1, 6144, 1024, 1, 2, 2, 16, 1, true, 8},
     {1, 151936, 1024, 0, 4, 2, 4, 1, false, 8},
-    // Gemma-style 12B (sandwich norms), 9-row verify: qkv 8.0 (8.4), o 5.2 (5.81), gate_up 23.6 (25.7),
+    // Gemma-style 12B (sandwich norms), 9-row verify: o 5.41 (5.81), gate_up 24.2 (25.7),
     // down 13.0 (14.3), head 176.4 (179.6)
-    {1, 8192, 3840, 2, 2, 1, 8, 1, true, 8},
-    {1, 3840, 4096, 2, 2, 2, 8, 2, true, 8},
-    {1, 30720, 3840, 1, 4, 2, 4, 1, true, 8},
+    {1, 3840, 4096, 2, 2, 2, 8, 2, false, 8},
+    {1, 30720, 3840, 1, 4, 2, 8, 1, false, 8},
     {1, 3840, 15360, 2, 2, 2, 8, 2, false, 8},
     {1, 262144, 3840, 0, 4, 2, 8, 1, false, 8},
+    // Qwen3-8B, 17-row verify (16 drafts and the bonus row): qkv 9.52 (10.13), gate_up 30.4 (33.3)
+    {2, 6144, 4096, 2, 2, 2, 8, 4, false, 8},
+    {2, 24576, 4096, 1, 2, 2, 8, 1, false, 8},
+    // Qwen3-8B, 36-row batch: qkv 11.85 (12.46)
+    {3, 6144, 4096, 2, 2, 2, 4, 4, false, 8},
     // 4-bit DFlash drafter of the Qwen3-8B shape: 16 block rows o 7.22 (7.76), gate_up 16.82
     // (19.09), down 10.67 (12.61); 17 context rows fc 20.76 (22.14), k|v 7.33 (8.10)
     {1, 4096, 4096, 2, 4, 2, 4, 8, true, 4},
@@ -828,22 +816,11 @@ static GemmPlan plan_gemm(int M, int64_t N, int64_t K, int epi, int bits = 8) {
     p.gpb = G;
     const int64_t nb = G / p.u;
     p.waves = nb >= 16 ? 16 : (nb >= 8 ? 8 : 4);
-    // more than one row tile (a sweep at M = 17, 36, 64 over o 4096x4096 and down 4096x12288):
-    // 8 waves of pipelined 2-group batches at two and four tiles (down 19.6 -> 18.7 and 30.6 -> 27.9 us
-    // against unpipelined ones), 16 waves of 4-group batches at three
-    p.pf = false;
-    if ((MT == 2 || MT == 4) && p.waves >= 8) {
-      p.waves = 8;
-      p.pf = true;
-    }
-    // short K at one tile (o 1024x2048, down 1024x3072 at M = 9): 8 waves of pipelined 4-group batches,
-    // 4.4 and 5.1 us against 4.5 and 5.3
-    if (MT == 1 && bits == 8 && G < 64 && G >= 32 && G % 4 == 0) {
-      p.u = 4;
-      p.waves = 8;
-      p.pf = true;
-    }
+    // more than one row tile (a sweep at M = 24, 36, 64 over o 4096x4096 and down 4096x12288):
+    // 8 waves of 2-group batches at two and four tiles, 16 waves of 4-group batches at three
+    if ((MT == 2 || MT == 4) && p.waves > 8) p.waves = 8;
     while ((size_t)p.waves * MT * 1024 > 65536) p.waves /= 2;
+    p.pf = false;  // pipelined loads measured slower here (down 4096x12288: 18.5 -> 23.2 us)
     return p;
   }
   p.u = 2;
@@ -889,41 +866,27 @@ static GemmPlan plan_gemm(int M, int64_t N, int64_t K, int epi, int bits = 8) {
     p.pf = true;
   }
   if (MT == 1 && bits == 8 && epi == DSK_EPI_STORE && tiles >= 4096 && G >= 64 && p.nt == 4) p.waves = 8;
-  // more than one row tile, from sweeps at M = 17, 20, 36 and 64 over the Qwen3-8B, Qwen3-0.6B and
-  // Gemma-style 12B shapes. The activation rows read per weight byte and the scaling grow with M, and
-  // batches of one group (fewer registers, more waves per SIMD) and wide slabs won:
-  //  - plain stores: slabs of 4 tiles, 4 waves (head 151936x4096: 143 -> 131 us at M = 17, 200 -> 181 at
-  //    36, 356 -> 235 at 64, each against 2-group batches);
-  //  - gated: the same for wide projections, pipelined at three tiles (gate_up 24576x4096: 40.8 -> 37.5
-  //    at 36, 61.6 -> 46.8 at 64; 30720x3840: 40.2 -> 31.4 at 36), pairs of tiles for narrow ones
-  //    (6144x1024 at M = 20: 8.6 -> 5.7);
-  //  - partial sums: K splits up to about 200 slabs (whole K ranges left a Gemma-style down 3840x15360
-  //    on 120 of 256 CUs: 36.7 -> 16.8 us at M = 36; o 3840x4096 11.9 -> 7.8; qkv 6144x4096 11.8 -> 10.6).
+  // more than one row tile, from a sweep at M = 24, 36 and 64 over the Qwen3-8B verify shapes
+  // (the 16-row rules above stay as fitted): the activation rows read per weight byte grow with
+  // M, and the plans that won keep whole K ranges and wide slabs. Partial sums: pairs of tiles,
+  // no K split, 16 waves at two tiles, 8 above (qkv 6144x4096 at M = 36: 27.2 -> 17.6 us); gated:
+  // 8 waves at four tiles (gate_up 24576x4096 at M = 64: 72.1 -> 63.6 us); plain stores (the
+  // logits): slabs of 4 tiles at two and three (head 151936x4096 at M = 36: 223.5 -> 192.4 us).
   if (MT >= 2 && bits == 8) {
-    p.u = 1;
-    p.sk = 1;
     if (partial) {
-      p.nt = MT <= 3 && G >= 32 && tiles % 4 == 0 ? 4 : 2;
-      p.waves = MT == 3 && p.nt == 4 ? 4 : 8;
-      p.pf = MT == 3 || (MT == 2 && p.nt == 2);
-      const int64_t want = p.nt == 4 ? 192 : (MT == 4 ? 512 : 256);
-      while (tiles / p.nt * p.sk < want && p.sk < (p.nt == 4 ? 8 : 4) && G / (p.sk * 2) >= p.waves) p.sk *= 2;
-    } else if (gated && tiles < 1024) {
-      p.nt = 2;
-      p.waves = MT == 2 ? 16 : 8;
-      p.pf = MT <= 3;
-    } else {
-      p.nt = 4;
-      p.waves = 4;
-      p.pf = gated && MT == 3;
-    }
-    if (tiles % p.nt) {  // slabs that divide: pairs (2-group batches where no 1-group kernel is built), tiles
-      p.nt = tiles % 2 ? 1 : 2;
+      p.nt = tiles % 2 == 0 ? 2 : 1;
+      p.sk = 1;
       p.u = 2;
+      p.gpb = G;
+      p.waves = MT == 2 ? 16 : 8;
+    } else if (gated) {
+      p.waves = MT >= 4 ? 8 : p.waves;
+    } else if (MT <= 3 && tiles % 4 == 0) {
+      p.nt = 4;
+      p.u = 2;
+      p.gpb = G;
       p.waves = 4;
-      p.pf = false;
     }
-    p.gpb = ((G / p.u + p.sk - 1) / p.sk) * p.u;
   }
   while ((size_t)p.waves * MT * p.nt * 1024 > 65536) p.waves /= 2;  // LDS of the reduction
   // 4-bit codes: a wave's load of one tile-group is 512 B, half the 8-bit one. Where the waves
@@ -973,22 +936,22 @@ static bool launch_gemm_w(const GemmArgs& a, int waves, hipStream_t st) {
 
 template <int BITS>
 static bool launch_gemm_bits(const GemmArgs& a, int MT, const GemmPlan& p, hipStream_t st) {
-#define DSK_GEMM_CASE(MT_, NT_, U_, PF_) \
-  if (MT == MT_ && p.nt == NT_ && p.u == U_ && p.pf == PF_) return launch_gemm_w<MT_, NT_, U_, PF_, BITS>(a, p.waves, st);
-  // pipelined
-  DSK_GEMM_CASE(1, 1, 2, true) DSK_GEMM_CASE(1, 2, 2, true) DSK_GEMM_CASE(1, 4, 2, true) DSK_GEMM_CASE(1, 1, 4, true)
-  DSK_GEMM_CASE(1, 2, 4, true) DSK_GEMM_CASE(1, 2, 1, true)
-  DSK_GEMM_CASE(2, 1, 2, true) DSK_GEMM_CASE(2, 2, 1, true)
-  DSK_GEMM_CASE(3, 2, 1, true) DSK_GEMM_CASE(3, 4, 1, true)
-  DSK_GEMM_CASE(4, 1, 2, true)
-  // a batch at a time
-  DSK_GEMM_CASE(1, 1, 2, false) DSK_GEMM_CASE(1, 2, 2, false) DSK_GEMM_CASE(1, 4, 2, false)
-  DSK_GEMM_CASE(1, 3, 2, false) DSK_GEMM_CASE(1, 6, 2, false) DSK_GEMM_CASE(1, 8, 2, false)
-  DSK_GEMM_CASE(1, 1, 4, false) DSK_GEMM_CASE(1, 2, 4, false) DSK_GEMM_CASE(1, 4, 4, false)
-  DSK_GEMM_CASE(2, 1, 2, false) DSK_GEMM_CASE(2, 2, 2, false) DSK_GEMM_CASE(2, 4, 2, false) DSK_GEMM_CASE(2, 4, 1, false)
-  DSK_GEMM_CASE(3, 1, 2, false) DSK_GEMM_CASE(3, 2, 2, false) DSK_GEMM_CASE(3, 4, 2, false) DSK_GEMM_CASE(3, 1, 4, false)
-  DSK_GEMM_CASE(3, 4, 1, false)
-  DSK_GEMM_CASE(4, 1, 2, false) DSK_GEMM_CASE(4, 2, 2, false) DSK_GEMM_CASE(4, 2, 1, false) DSK_GEMM_CASE(4, 4, 1, false)
+  if (p.pf) {  // the pipelined variant is built for the shapes the planner gives it
+    if (MT == 1 && p.nt == 2 && p.u == 2) return launch_gemm_w<1, 2, 2, true, BITS>(a, p.waves, st);
+    if (MT == 1 && p.nt == 2 && p.u == 4) return launch_gemm_w<1, 2, 4, true, BITS>(a, p.waves, st);
+    if (MT == 1 && p.nt == 4 && p.u == 2) return launch_gemm_w<1, 4, 2, true, BITS>(a, p.waves, st);
+    if (MT == 1 && p.nt == 1 && p.u == 4) return launch_gemm_w<1, 1, 4, true, BITS>(a, p.waves, st);
+    if (MT == 1 && p.nt == 1 && p.u == 2) return launch_gemm_w<1, 1, 2, true, BITS>(a, p.waves, st);
+    return false;
+  }
+#define DSK_GEMM_CASE(MT_, NT_, U_) \
+  if (MT == MT_ && p.nt == NT_ && p.u == U_) return launch_gemm_w<MT_, NT_, U_, false, BITS>(a, p.waves, st);
+  DSK_GEMM_CASE(1, 1, 2) DSK_GEMM_CASE(1, 2, 2) DSK_GEMM_CASE(1, 4, 2) DSK_GEMM_CASE(1, 8, 2)
+  DSK_GEMM_CASE(1, 3, 2) DSK_GEMM_CASE(1, 6, 2)
+  DSK_GEMM_CASE(1, 1, 4) DSK_GEMM_CASE(1, 2, 4) DSK_GEMM_CASE(1, 4, 4)
+  DSK_GEMM_CASE(2, 1, 2) DSK_GEMM_CASE(2, 2, 2) DSK_GEMM_CASE(2, 4, 2)
+  DSK_GEMM_CASE(3, 1, 2) DSK_GEMM_CASE(3, 2, 2) DSK_GEMM_CASE(3, 4, 2) DSK_GEMM_CASE(3, 1, 4)
+  DSK_GEMM_CASE(4, 1, 2) DSK_GEMM_CASE(4, 2, 2)
 #undef DSK_GEMM_CASE
   return false;
 }
@@ -1234,7 +1197,7 @@ extern "C" int dsk_w8_gemm_rn_planned(const uint16_t* xp, const uint8_t* wt, con
   const int MT = (M + 15) / 16;
   DSK_REQUIRE(slab_tiles >= 1 && slab_tiles <= 8 && N % 16 == 0 && tiles % slab_tiles == 0,
               "%s: %d tiles per slab do not divide N / 16 = %lld", who, slab_tiles, (long long)tiles);
-  DSK_REQUIRE((batch_groups == 1 || batch_groups == 2 || batch_groups == 4) && K % 64 == 0 && G % batch_groups == 0,
+  DSK_REQUIRE((batch_groups == 2 || batch_groups == 4) && K % 64 == 0 && G % batch_groups == 0,
               "%s: batches of %d groups", who, batch_groups);
   DSK_REQUIRE(waves == 4 || waves == 8 || waves == 16, "%s: %d waves", who, waves);
   DSK_REQUIRE(k_splits >= 1 && (k_splits == 1 || epi == DSK_EPI_PARTIAL) && k_splits <= G / batch_groups,
