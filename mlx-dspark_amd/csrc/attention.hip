@@ -182,10 +182,20 @@ __global__ __launch_bounds__(256) void qkv_rope_append_rows_kernel(
     for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32(h16[e]);
     const bool is_q = head < nq, is_k = !is_q && head < nq + nkv;
     const uint16_t* nw = is_q ? q_norm : (is_k ? k_norm : v_norm);
-    float ss = 0.0f;
+    // summed as norm_rope_row<HD, 64> does (a wave's lane there holds HD / 64 dims): the same bits
+    constexpr int P = HD / 64;
+    float sp[8 / P];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-    ss = row_sum<L>(ss);
+    for (int i = 0; i < 8 / P; ++i) {
+      sp[i] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < P; ++e) sp[i] += v[i * P + e] * v[i * P + e];
+    }
+#pragma unroll
+    for (int o = 1; o < 8 / P; o <<= 1)
+#pragma unroll
+      for (int i = 0; i + o < 8 / P; i += 2 * o) sp[i] += sp[i + o];
+    const float ss = row_sum<L>(sp[0]);
     if (nw) {
       const float r = rsqrtf(ss / (float)HD + eps);
       const u32x4 gw = *reinterpret_cast<const u32x4*>(nw + sub * 8);

@@ -214,6 +214,29 @@ def test_append_of_many_rows_equals_the_general_form(dev, hd, nq, nkv, kv_bits, 
         assert float((ka[i] != kb[i]).float().mean()) < 0.02
 
 
+@pytest.mark.parametrize("hd,nq,nkv,kv_bits,B,W", [
+    (128, 32, 8, 8, 1, 4096), (128, 5, 1, None, 2, 515), (256, 16, 8, None, 1, 2048), (512, 3, 1, 8, 1, 700),
+])
+def test_append_of_many_rows_has_the_general_forms_bits(dev, hd, nq, nkv, kv_bits, B, W):
+    """The norm's float32 sums are taken in the order of the wave-per-head form: the same queries, keys,
+    values and scales, bit for bit (another order flips a few of a million roundings)."""
+    from mlx_dspark import ops
+    from mlx_dspark.kv import PagedKVCache
+    print(f"append bits hd={hd} nq={nq} nkv={nkv} kv_bits={kv_bits} B={B} W={W}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(hd + W)
+    qkv = (torch.randn(B * W, (nq + 2 * nkv) * hd, generator=g, device=dev) * 2).to(torch.bfloat16)
+    gains = [(1 + 0.2 * torch.randn(hd, generator=g, device=dev)).to(torch.bfloat16) for _ in range(3)]
+    inv = ops.rope_inv_freq(hd, 1e6, dev)
+    outs = []
+    for x in (qkv, qkv.float()[None]):
+        cache = PagedKVCache(1, B, nkv, hd, W + 100, kv_bits=kv_bits)
+        cache.set_lengths([37 * b + 5 for b in range(B)])
+        q = ops.qkv_rope_append(x.contiguous(), B, W, nq, nkv, hd, gains[0], gains[1], 1e-6, inv, cache.seq_lens,
+                                cache.block_table, cache.page, cache.kv_dtype, *cache.layer_args(0), v_norm=gains[2])
+        outs.append([q] + [t for t in cache.layer_args(0) if t is not None])
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
 @pytest.mark.parametrize("n,H", [(1, 64), (3, 1024), (130, 4096)])
 def test_embed_in_whole_pieces_equals_the_general_form(dev, n, H):
     """16 codes per thread (aligned rows and outputs) against one element per thread (an output row
