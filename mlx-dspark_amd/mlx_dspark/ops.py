@@ -351,6 +351,7 @@ class Rows:
 
 
 ROWS_MAX_K = 24576   # widest rows dsk_rows_prep holds in registers
+ROWS_MAX_PAGES = 1024   # pages per row dsk_attention_rows keeps the ids of in LDS
 
 
 def rows_prep(h: torch.Tensor, *, norm_w: torch.Tensor | None = None, eps: float = 0.0, later: bool = False,
@@ -500,11 +501,17 @@ def attention(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page,
 
 
 
+def attention_rows_takes(hd: int, max_pages: int) -> bool:
+    """Whether dsk_attention_rows takes a head_dim and a block table's width."""
+    return hd in (128, 256) and max_pages <= ROWS_MAX_PAGES
+
+
 def attention_rows(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page, kv_dtype, k_pool, v_pool,
                    k_sb=None, v_sb=None, *, causal=True, window=0):
     """attention of a prompt's many rows, bf16 [B*W, nq*hd], with the verify kernels' float32
-    probabilities (dsk_attention_rows; dsk_attention where its shapes end)."""
-    if hd not in (128, 256) or block_table.shape[1] > 1024:
+    probabilities (dsk_attention_rows; dsk_attention where its shapes end, with scratch for every row and
+    key split: by attention_rows_takes a caller can give that one fewer rows at a time)."""
+    if not attention_rows_takes(hd, block_table.shape[1]):
         return attention(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page, kv_dtype, k_pool, v_pool,
                          k_sb, v_sb, causal=causal, window=window)
     out = torch.empty((B * W, nq * hd), dtype=torch.bfloat16, device=q.device)

@@ -32,6 +32,12 @@ from .ops import DSK_EPI_GEGLU, DSK_EPI_SWIGLU, W8Table, W8Weight
 MAX_ROWS = 64  # rows per kernel pass (M of the skinny GEMM)
 DENSE_MIN_ROWS = 256   # prompts from this length prefill layer by layer through the library GEMM
 PREFILL_CHUNK = 2048   # prompt rows handed to a drafter per on_chunk call (generate.py:613-656)
+# Prompt rows per pass where the attention splits the keys (block tables of more than 1024 pages: 65536
+# positions in pages of 64): its scratch is rows x splits of the whole table, kept for good, half of a
+# 64-row pass's at 256 rows (2048 rows of 16 heads of 256 over 131072 positions: 8.7 GB). 1027 tokens into
+# such a cache, two Qwen3-8B layers: 6.7 ms in 64-row passes, 5.8 in pieces of 256, 7.0 in one; six
+# Gemma-style ones 25.0, 17.4 and 17.1.
+SPLIT_CHUNK = 256
 
 
 @dataclass
@@ -299,8 +305,9 @@ class Qwen3W8:
         [1, L, n_tap*H] or None). on_chunk(fused_chunk, pos) lets a drafter ingest the hidden
         states chunk by chunk. A Qwen3-layout prompt of DENSE_MIN_ROWS rows or more runs layer
         by layer over all its rows (prefill_dense). Others (or dense=False) run in pieces of up to
-        PREFILL_CHUNK rows whose projections keep the codes' own arithmetic (_rows_pass), with a last
-        piece of at most MAX_ROWS rows (or every piece, when ``chunk`` is smaller) in a forward pass."""
+        PREFILL_CHUNK rows (SPLIT_CHUNK over very long caches) whose projections keep the codes' own
+        arithmetic (_rows_pass), with a last piece of at most MAX_ROWS rows (or every piece, when
+        ``chunk`` is smaller) in a forward pass."""
         if not torch.is_tensor(ids):
             ids = torch.tensor(ids, dtype=torch.int32)
         ids = ids.reshape(1, -1).to(self.device, torch.int32)
@@ -313,7 +320,7 @@ class Qwen3W8:
         parts = []
         out = None
         pos = cache.lengths[0]
-        piece = PREFILL_CHUNK if chunk == MAX_ROWS and self._rows_ok else chunk
+        piece = self._rows_piece(cache) if chunk == MAX_ROWS and self._rows_ok else chunk
         for c0 in range(0, L, piece):
             c1 = min(L, c0 + piece)
             last = c1 == L
@@ -338,6 +345,11 @@ class Qwen3W8:
         a = self.args
         return all(k % 256 == 0 and k <= ops.ROWS_MAX_K
                    for k in (a.hidden_size, a.num_attention_heads * a.head_dim, a.intermediate_size))
+
+    def _rows_piece(self, cache: PagedKVCache) -> int:
+        """Rows of one _rows_pass over this cache."""
+        takes = ops.attention_rows_takes(self.args.head_dim, cache.block_table.shape[1])
+        return PREFILL_CHUNK if takes else SPLIT_CHUNK
 
     def _rows_pass(self, ids: torch.Tensor, cache: PagedKVCache, tap=None, *, logits: str = "last"):
         """forward over one row of more than MAX_ROWS new tokens, with its rounding points: row-major

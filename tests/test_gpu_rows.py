@@ -171,6 +171,27 @@ def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
         assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
 
 
+def test_prompt_into_a_very_long_cache_keeps_small_scratch(dev, monkeypatch):
+    """A block table wider than the many-row attention takes: the split attention's scratch stays within
+    a 64-row pass's, and the results are those of 64-row passes (rounding flips: 2e-2 of the largest)."""
+    from mlx_dspark import _hip, ops, synthetic
+    model = synthetic.build_target("tiny-gemma", seed=43)
+    a, pages, n = model.args, ops.ROWS_MAX_PAGES + 1, 600
+    prompt = torch.randint(0, a.vocab_size, (n,), generator=torch.Generator().manual_seed(2)).tolist()
+    reserve, asked = ops.Workspace.reserve, []
+    monkeypatch.setattr(ops.Workspace, "reserve",
+                        lambda self, kind, b: (asked.append(b) if kind == "attn" else None, reserve(self, kind, b))[1])
+    outs = []
+    for chunk in (64, 63):           # 63: forward passes
+        cache = model.make_cache(max_ctx=pages * 64)
+        assert cache.block_table.shape[1] == pages
+        logits, fused = model.prefill(prompt, cache, [0, 5], chunk=chunk)
+        outs.append((logits, fused))
+    assert max(asked) <= _hip.lib.dsk_attn_ws_bytes(1, 64, a.num_attention_heads, a.head_dim, pages * 64)
+    for x, y in zip(*outs):
+        assert float((x.float() - y.float()).abs().max()) <= 2e-2 * float(y.float().abs().max())
+
+
 @pytest.mark.parametrize("hd,nq,nkv,kv_bits,v_norm,B,W", [
     (128, 4, 2, None, False, 1, 203), (128, 0, 3, 8, False, 2, 70), (128, 5, 1, 8, True, 1, 128),
     (256, 4, 2, 8, False, 1, 131), (256, 2, 1, None, True, 3, 50), (512, 3, 1, 8, True, 1, 130),
