@@ -306,8 +306,9 @@ class Qwen3W8:
         states chunk by chunk. A Qwen3-layout prompt of DENSE_MIN_ROWS rows or more runs layer
         by layer over all its rows (prefill_dense). Others (or dense=False) run in pieces of up to
         PREFILL_CHUNK rows (SPLIT_CHUNK over very long caches) whose projections keep the codes' own
-        arithmetic (_rows_pass), with a last piece of at most MAX_ROWS rows (or every piece, when
-        ``chunk`` is smaller) in a forward pass."""
+        arithmetic (_rows_pass), with a last piece of at most MAX_ROWS rows in a forward pass. That is
+        the default ``chunk`` of MAX_ROWS; another number is the rows of every forward pass, which takes
+        at most MAX_ROWS."""
         if not torch.is_tensor(ids):
             ids = torch.tensor(ids, dtype=torch.int32)
         ids = ids.reshape(1, -1).to(self.device, torch.int32)
@@ -320,11 +321,12 @@ class Qwen3W8:
         parts = []
         out = None
         pos = cache.lengths[0]
-        piece = self._rows_piece(cache) if chunk == MAX_ROWS and self._rows_ok else chunk
+        many = chunk == MAX_ROWS and self._rows_ok
+        piece = self._rows_piece(cache) if many else chunk
         for c0 in range(0, L, piece):
             c1 = min(L, c0 + piece)
             last = c1 == L
-            run = self._rows_pass if c1 - c0 > MAX_ROWS else self.forward
+            run = self._rows_pass if many and c1 - c0 > MAX_ROWS else self.forward
             out, fused = run(ids[:, c0:c1], cache, tap, logits="last" if last else "none")
             if fused is not None:
                 if on_chunk is not None:

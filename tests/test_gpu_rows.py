@@ -171,6 +171,21 @@ def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
         assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
 
 
+def test_prompt_pieces_wider_than_a_forward_pass_are_refused(dev):
+    """An explicit chunk of more than 64 rows, before any key is appended; a prompt that fits one pass is
+    taken whatever the chunk."""
+    from mlx_dspark import synthetic
+    model = synthetic.build_target("tiny", seed=44)
+    cache = model.make_cache(max_ctx=320)
+    for chunk in (65, 128, 2048):
+        with pytest.raises(ValueError, match="rows per batch row"):
+            model.prefill(list(range(200)), cache, None, chunk=chunk)
+    torch.cuda.synchronize()
+    assert cache.lengths[0] == 0 and not any(bool(k.any()) for k in cache.k)
+    model.prefill(list(range(50)), cache, None, chunk=128)
+    assert cache.lengths[0] == 50
+
+
 def test_prompt_into_a_very_long_cache_keeps_small_scratch(dev, monkeypatch):
     """A block table wider than the many-row attention takes: the split attention's scratch stays within
     a 64-row pass's, and the results are those of 64-row passes (rounding flips: 2e-2 of the largest)."""
