@@ -384,13 +384,21 @@ __device__ __forceinline__ float yv(float x, int mul, float T, float inv_t) {
 }
 __device__ __forceinline__ uint32_t samp_offset(const SampArgs& a) { return a.offset_dev ? a.offset_dev[0] : a.offset; }
 
-// the row's max from its slices', a lane per slice: every lane of the calling wave takes part (one
-// round trip); few slices are read in turn
+// the row's max from its slices'. More than kTurnSlices of them (WIDE): a lane per slice, every lane of
+// the calling wave takes part (18 rows at 32 slices: 54.2 -> 52.4 us a sampled acceptance). Few are read
+// in turn by scalar loads, which do not queue behind the slice's own vector loads. Each kernel is
+// compiled for one form: with both behind a branch the gather and stats passes of the 132 rows of a
+// 4 x 16 acceptance each lost 0.2-0.4 us (83.9 against 83.1 us).
+constexpr int kTurnSlices = 16;
+template <bool WIDE>
 __device__ __forceinline__ float row_max(const SampArgs& a, int r) {
-  if (a.S > 16) return wave_max(a.gmax[r * kMaxSlices + min((int)(threadIdx.x & 63), a.S - 1)]);
-  float m = a.gmax[r * kMaxSlices];
-  for (int s = 1; s < a.S; ++s) m = fmaxf(m, a.gmax[r * kMaxSlices + s]);
-  return m;
+  if constexpr (WIDE) {
+    return wave_max(a.gmax[r * kMaxSlices + min((int)(threadIdx.x & 63), a.S - 1)]);
+  } else {
+    float m = a.gmax[r * kMaxSlices];
+    for (int s = 1; s < a.S; ++s) m = fmaxf(m, a.gmax[r * kMaxSlices + s]);
+    return m;
+  }
 }
 
 // final probability of element j of a row with parameters rp
@@ -513,7 +521,7 @@ __global__ __launch_bounds__(kST) void samp_max_kernel(SampArgs a) {
 // ---- pass 2: Z and the first-level histogram, merged per row by integer atomics. Lanes
 // spread their LDS atomics over kHistCopies copies (copy = lane % kHistCopies) so lanes of one
 // wave that hit the same bucket mostly hit different addresses.
-template <bool VEC, bool TONE>
+template <bool VEC, bool TONE, bool WIDE>
 __global__ __launch_bounds__(kST) void samp_stats_kernel(SampArgs a) {
   __shared__ uint32_t hc[kHistCopies][kL1 + 1];  // +1: copies start in different LDS banks
   __shared__ unsigned long long hw[kHistCopies][kL1 + 1];
@@ -526,7 +534,7 @@ __global__ __launch_bounds__(kST) void samp_stats_kernel(SampArgs a) {
   const int64_t lo = min(a.V, (int64_t)s * a.slen), hi = min(a.V, lo + a.slen);
   SliceRegs<VEC> xr;
   xr.load(x, lo, hi);  // in flight while the row max is read and the histogram cleared
-  const float m = row_max(a, r);
+  const float m = row_max<WIDE>(a, r);
   uint32_t* hcp = hc[threadIdx.x % kHistCopies];
   unsigned long long* hwp = hw[threadIdx.x % kHistCopies];
   if (trunc) {
@@ -599,12 +607,13 @@ struct SelSmem {
 // gather 8.0 us in two launches, 9.8 in one; the whole chain of seven draws 343 -> 313 us, together
 // with 64 slices instead of 32). With 12 rows at 64 slices the smaller slices' fixed costs (histogram
 // merge, clears) lost 20 %, and with 132 rows the repeated selection 3 %: those keep the two launches.
+template <bool WIDE>
 __device__ RowInfo select_row(const SampArgs& a, int r, SelSmem& sm) {
   const uint64_t Z = a.zsum[r];
   const int bb = kL1 - 1 - (int)threadIdx.x;
   const uint64_t c = a.hcnt[r * kL1 + bb];
   const uint64_t w = a.hwgt[r * kL1 + bb];
-  const float m = row_max(a, r);
+  const float m = row_max<WIDE>(a, r);
   const uint64_t TP = a.do_p ? top_p_target(a.top_p, Z) : 0;
   if (threadIdx.x == 0) {
     sm.sel[0] = kNone;
@@ -648,16 +657,17 @@ __device__ RowInfo select_row(const SampArgs& a, int r, SelSmem& sm) {
   return sm.info;
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(kST) void samp_select_kernel(SampArgs a) {
   __shared__ SelSmem sm;
-  const RowInfo inf = select_row(a, blockIdx.x, sm);
+  const RowInfo inf = select_row<WIDE>(a, blockIdx.x, sm);
   if (threadIdx.x == 0) a.info[blockIdx.x] = inf;
 }
 
 // ---- pass 3b (truncation): the candidates of the threshold buckets. A cheap window test
 // stages each wave's window elements in LDS by ballot; the exact keys of the staged elements are
 // then computed densely, so exp never runs divergently.
-template <bool VEC, bool TONE, bool SEL>
+template <bool VEC, bool TONE, bool SEL, bool WIDE>
 __global__ __launch_bounds__(kST) void samp_gather_kernel(SampArgs a) {
   __shared__ uint64_t sh[kSW];
   __shared__ uint32_t base[2];
@@ -673,12 +683,12 @@ __global__ __launch_bounds__(kST) void samp_gather_kernel(SampArgs a) {
   RowInfo inf;
   if constexpr (SEL) {  // few rows: every workgroup selects for itself, one launch less
     __shared__ SelSmem sm;
-    inf = select_row(a, r, sm);
+    inf = select_row<WIDE>(a, r, sm);
     if (s == 0 && threadIdx.x == 0) a.info[r] = inf;
   } else {
     inf = a.info[r];
   }
-  const float m = row_max(a, r);
+  const float m = row_max<WIDE>(a, r);
   const uint32_t bk = inf.bk, bq = (inf.bp == inf.bk) ? kNone : inf.bp;
   if (bk == kNone && bq == kNone) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -801,11 +811,12 @@ __device__ uint64_t mass_at_or_above(const uint32_t* cand, uint32_t n, uint32_t 
   return block_sum512(t, sm.sh);
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(kST) void samp_finish_kernel(SampArgs a) {
   __shared__ FinSmem sm;
   const int r = blockIdx.x;
   RowParam rp;
-  rp.m = row_max(a, r);
+  rp.m = row_max<WIDE>(a, r);
   rp.pad = 0;
   const uint64_t Z = a.zsum[r];
   if (!a.do_k && !a.do_p) {
@@ -1159,28 +1170,35 @@ static int launch_sampled(SampArgs& a, int draws, hipStream_t st, const char* wh
   const dim3 grow((unsigned)(rows * a.S));
   const bool one = a.T == 1.0f;
   const bool few = rows <= kFewRows;
-#define DSK_ROW_PASSES(VEC_, ONE_)                                                 \
-  hipLaunchKernelGGL((samp_max_kernel<VEC_, ONE_>), grow, blk, 0, st, a);          \
-  hipLaunchKernelGGL((samp_stats_kernel<VEC_, ONE_>), grow, blk, 0, st, a);        \
-  if (a.do_k || a.do_p) {                                                          \
-    if (few) {                                                                     \
-      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, true>), grow, blk, 0, st, a);  \
-    } else {                                                                       \
-      hipLaunchKernelGGL(samp_select_kernel, dim3((unsigned)rows), blk, 0, st, a); \
-      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, false>), grow, blk, 0, st, a); \
-    }                                                                              \
+#define DSK_ROW_PASSES(VEC_, ONE_, WIDE_)                                                      \
+  hipLaunchKernelGGL((samp_max_kernel<VEC_, ONE_>), grow, blk, 0, st, a);                      \
+  hipLaunchKernelGGL((samp_stats_kernel<VEC_, ONE_, WIDE_>), grow, blk, 0, st, a);             \
+  if (a.do_k || a.do_p) {                                                                      \
+    if (few) {                                                                                 \
+      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, true, true>), grow, blk, 0, st, a);   \
+    } else {                                                                                   \
+      hipLaunchKernelGGL((samp_select_kernel<WIDE_>), dim3((unsigned)rows), blk, 0, st, a);    \
+      hipLaunchKernelGGL((samp_gather_kernel<VEC_, ONE_, false, WIDE_>), grow, blk, 0, st, a); \
+    }                                                                                          \
+  }                                                                                            \
+  hipLaunchKernelGGL((samp_finish_kernel<WIDE_>), dim3((unsigned)rows), blk, 0, st, a);
+#define DSK_ROW_WIDTH(VEC_, ONE_)      \
+  if (a.S > kTurnSlices) {             \
+    DSK_ROW_PASSES(VEC_, ONE_, true)   \
+  } else {                             \
+    DSK_ROW_PASSES(VEC_, ONE_, false)  \
   }
   if (a.vec && one) {
-    DSK_ROW_PASSES(true, true)
+    DSK_ROW_WIDTH(true, true)
   } else if (a.vec) {
-    DSK_ROW_PASSES(true, false)
+    DSK_ROW_WIDTH(true, false)
   } else if (one) {
-    DSK_ROW_PASSES(false, true)
+    DSK_ROW_WIDTH(false, true)
   } else {
-    DSK_ROW_PASSES(false, false)
+    DSK_ROW_WIDTH(false, false)
   }
+#undef DSK_ROW_WIDTH
 #undef DSK_ROW_PASSES
-  hipLaunchKernelGGL(samp_finish_kernel, dim3((unsigned)rows), blk, 0, st, a);
   hipLaunchKernelGGL(samp_wsum_kernel, dim3((unsigned)(draws * a.Sd)), blk, 0, st, a);
   hipLaunchKernelGGL(samp_draw_kernel, dim3((unsigned)draws), blk, 0, st, a);
   DSK_LAUNCH_CHECK(who);

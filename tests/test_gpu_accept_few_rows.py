@@ -1,5 +1,6 @@
 """GPU parity of row sampling on both sides of the few-rows rule (up to four rows the gather pass
-finds the threshold buckets itself and rows are cut into up to 64 slices): tokens and probabilities
+finds the threshold buckets itself and rows are cut into up to 64 slices) and of 16 slices per row
+(their maxima read a lane each beyond, in turn up to it): tokens and probabilities
 bit-identical to the oracle for every truncation, at vocabularies of one slice, of slices that do
 not divide, and unaligned ones, with heavy ties and an all-equal row."""
 
@@ -12,7 +13,8 @@ from oracle import accept as A
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("R,V", [(1, 511), (1, 151936), (3, 33001), (4, 40960), (4, 32771), (5, 40960), (17, 9001)])
+@pytest.mark.parametrize("R,V", [(1, 511), (1, 151936), (3, 33001), (4, 40960), (4, 32771), (5, 40960), (17, 9001),
+                                 (70, 9001)])
 @pytest.mark.parametrize("T,tp,tk", [(1.0, 0.9, 0), (0.7, 1.0, 20), (0.8, 0.95, 50), (1.0, 0.0, 0), (0.5, 1.0, 0)])
 def test_sample_rows_few(dev, R, V, T, tp, tk):
     from mlx_dspark.ops import sample_rows
