@@ -676,6 +676,14 @@ def logits_penalize(logits: torch.Tensor, row_ptr: torch.Tensor, ids: torch.Tens
 
 
 # ----------------------------------------------------------------------------- logprobs
+# Rows are split over workgroups (dsk_row_logprobs_ws) from one slice's 4096 elements and this many element
+# reads (one pass and one per alternative): below, the second kernel and its scratch cost a call more than
+# they save. Back to back, one workgroup per row against the split: V = 1000 with 5 alternatives 17.8 and
+# 22.3 us, 32000 with none 17.9 and 22.4, 24000 with two 21.2 and 22.2; 4096 with 20 52.3 and 49.7, 48000
+# with one 25.2 and 22.4, 100000 with none 26.7 and 22.7.
+LOGPROBS_SPLIT_V, LOGPROBS_SPLIT_READS = 4096, 75_000
+
+
 def row_logprobs(logits: torch.Tensor, tokens: torch.Tensor, top_k: int = 0):
     """logits [R, V] f32 (unit column stride), tokens int32 [R] -> (chosen f32 [R], top_ids
     int32 [R, top_k], top_vals f32 [R, top_k]) of log_softmax(logits) (see dsk_row_logprobs)."""
@@ -687,8 +695,10 @@ def row_logprobs(logits: torch.Tensor, tokens: torch.Tensor, top_k: int = 0):
     chosen = torch.empty(R, dtype=torch.float32, device=dev)
     ids = torch.empty((R, max(top_k, 1)), dtype=torch.int32, device=dev)
     vals = torch.empty((R, max(top_k, 1)), dtype=torch.float32, device=dev)
-    need = _hip.lib.dsk_row_logprobs_ws_bytes(R, V, int(top_k))
-    if need == 0:   # shapes beyond the split form (or arguments the entry refuses)
+    need = 0
+    if V >= LOGPROBS_SPLIT_V and V * (top_k + 1) >= LOGPROBS_SPLIT_READS:
+        need = _hip.lib.dsk_row_logprobs_ws_bytes(R, V, int(top_k))
+    if need == 0:   # short rows, shapes beyond the split form (or arguments the entry refuses)
         call("dsk_row_logprobs", ptr(logits), logits.stride(0), R, V, ptr(tokens), int(top_k), ptr(chosen), ptr(ids),
              ptr(vals), stream_ptr())
     else:
