@@ -1960,12 +1960,18 @@ static int qkv_append_entry(const void* qkv, int qkv_splits, int B, int W, int n
   DSK_REQUIRE(!x_ssq || qkv_splits > 0, "dsk_qkv_rope_append_rn: the row scale applies to f32 split-K slices");
   DSK_REQUIRE(kv_dtype == DSK_KV_BF16 || (kv_dtype == DSK_KV_U8 && k_sb && v_sb),
               "dsk_qkv_rope_append: u8 KV needs scale/bias buffers");
-  // many rows: a workgroup per row instead of a wave per head. Below 128 rows the workgroups of a row
-  // leave half of the CUs idle; at 203 rows of 48 heads the two forms take 5.5 and 5.9 us.
-  if (qkv_splits == 0 && B * W >= 128 &&
+  // many rows: a workgroup per row instead of a wave per head, where that was no slower in a sweep of 1 to
+  // 48 heads and 128 to 2048 rows (us, wave per head / workgroup per row). From 2048 columns, which fill a
+  // workgroup's lanes, at 129 rows (48 heads of 128: 5.4 / 5.3, 128 rows 4.9 / 5.2), at 176 for 4096 and
+  // more columns in wide heads (32 of 256: 5.8 / 5.7, 160 rows 5.2 / 5.7); fewer columns leave lanes idle
+  // and need more rows for it (8 heads of 128: 3.1 / 3.2 at 256 rows, 3.5 / 3.3 at 384), and below four
+  // heads the general form stays ahead (2 heads of 128, 2048 rows: 3.7 / 4.3).
+  const int heads = nq + 2 * nkv, cols = heads * hd, rows = B * W;
+  const int min_rows = cols < 2048 ? 400000 / cols : (hd > 128 && cols >= 4096 ? 176 : 129);
+  if (qkv_splits == 0 && heads >= 4 && rows >= min_rows &&
       (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)q_norm | (uintptr_t)k_norm | (uintptr_t)v_norm |
         (uintptr_t)k_pool | (uintptr_t)v_pool) & 15) == 0) {
-    const dim3 rgrid((unsigned)(B * W));
+    const dim3 rgrid((unsigned)rows);
 #define DSK_APPEND_ROWS(HDV)                                                                                        \
   hipLaunchKernelGGL((qkv_rope_append_rows_kernel<HDV>), rgrid, dim3(256), 0, as_stream(stream),                    \
                      reinterpret_cast<const uint16_t*>(qkv), W, nq, nkv, q_norm, k_norm, v_norm, eps, inv_freq,     \
