@@ -1414,8 +1414,8 @@ constexpr int kPfMaxPages = 1024;             // page ids of a row block's keys 
 // staging and MFMAs interleave). On the 4096-token Qwen3-8B layer: 436 us with 4 waves and no bound, 299 us
 // with 4 waves and this bound, 239 us with 8 waves sharing each block's dequantisation (one bf16 term
 // of P); with two terms of P 326 us, 263 us (522 TFLOP/s) since the tokens are found once per key and
-// half the waves stage first. 4 waves of one tile where the 256-row blocks leave CUs idle, and at head_dim 256, where the
-// two K/V buffers fill the LDS.
+// half the waves stage first. 4 waves of one tile for few rows (prompt_blocks_small), and at head_dim
+// 256, where the two K/V buffers fill the LDS.
 // a loaded chunk as four words of two bf16 values
 template <int KVT>
 __device__ __forceinline__ u32x4 chunk_words(const Chunk8& c) {
@@ -1728,14 +1728,26 @@ static void launch_prompt_shape(const AttnArgs& a, hipStream_t st) {
   else
     hipLaunchKernelGGL((attention_prefill_kernel<HD, DSK_KV_BF16, TERMS, NW, TPW>), grid, blk, 0, st, a);
 }
+// Blocks of 64 query rows instead of 256 at head_dim 128. Two of their workgroups fit a CU, so up to 512
+// run at once, and with a quarter of the rows each ends sooner (us in 256-row and 64-row blocks, 32 heads
+// over 8 kv heads, 8-bit, after 4000 cached positions: 255 rows 255 and 181, 1000 rows 257 and 226). Past 512
+// a second round repeats every key's dequantisation (1100 rows: 261 and 353), except where the positions
+// before the prompt are few and the blocks' key ranges are a triangle, whose short ones fill the gaps (no
+// cached position: 1500 rows 86 and 72, 1920 rows 106 and 105), up to a 256-row block per CU.
+static bool prompt_blocks_small(const AttnArgs& a, int64_t max_ctx) {
+  const int64_t heads = (int64_t)a.B * a.nkv;
+  if (heads * ceil_div(a.R, 64) <= 512) return true;
+  return a.causal && heads * ceil_div(a.R, 256) < 256 && max_ctx - a.W <= a.W / 4;
+}
+// max_ctx bounds the positions of any row's keys
 template <int TERMS>
-static void launch_prompt_attention(AttnArgs& a, int hd, hipStream_t st) {
+static void launch_prompt_attention(AttnArgs& a, int hd, int64_t max_ctx, hipStream_t st) {
   a.nsplit = 1;
   a.part_o = nullptr;
   a.part_ml = nullptr;
   if constexpr (TERMS == 3)
     if (hd == 256) return launch_prompt_shape<256, TERMS, 4, 1>(a, st);
-  if ((int64_t)a.B * a.nkv * ceil_div(a.R, 256) < 256) return launch_prompt_shape<128, TERMS, 4, 1>(a, st);
+  if (prompt_blocks_small(a, max_ctx)) return launch_prompt_shape<128, TERMS, 4, 1>(a, st);
   launch_prompt_shape<128, TERMS, 8, 2>(a, st);
 }
 
@@ -1791,7 +1803,7 @@ static int attention_run(AttnArgs& a, int hd, int max_ctx, float softcap, void* 
   a.fused = fused ? 1 : 0;
   const bool sc = softcap > 0.0f;
   if (hd == 128 && !fused && !sc && !a.out_packed && a.W > kAttnVerifyMaxW && a.max_pages <= kPfMaxPages) {
-    launch_prompt_attention<2>(a, hd, st);
+    launch_prompt_attention<2>(a, hd, max_ctx, st);
     DSK_LAUNCH_CHECK(who);
     return DSK_OK;
   }
@@ -2096,7 +2108,7 @@ extern "C" int dsk_attention_rows(const uint16_t* q, int B, int W, int nq, int n
   a.k_sb = const_cast<uint32_t*>(k_sb);
   a.v_sb = const_cast<uint32_t*>(v_sb);
   a.out = out;
-  launch_prompt_attention<3>(a, hd, as_stream(stream));
+  launch_prompt_attention<3>(a, hd, (int64_t)max_pages * page, as_stream(stream));
   DSK_LAUNCH_CHECK(who);
   return DSK_OK;
 }

@@ -453,6 +453,10 @@ class Qwen3W8:
         qkv = torch.empty((L, a.n_qkv), dtype=torch.bfloat16, device=dev)
         gu = torch.empty((L, 2 * I), dtype=torch.bfloat16, device=dev)
         act = torch.empty((L, I), dtype=torch.bfloat16, device=dev)
+        # the many-query kernel takes max_ctx as a bound of the keys only to choose its blocks; the
+        # split one (other head_dims, very long caches) sizes its splits by it
+        bounded = hd == 128 and ops.attention_rows_takes(hd, cache.block_table.shape[1])
+        ctx = cache.lengths[0] + L if bounded else cache.max_ctx
         for l, Lw in enumerate(self.layers):
             ops.rows_rmsnorm(h, Lw.in_norm, eps, out=x)
             torch.matmul(x, rows(l, "qkv").t(), out=qkv)
@@ -460,7 +464,7 @@ class Qwen3W8:
             inv_freq = self.inv_freq_local if a.is_sliding(l) else self.inv_freq
             q = ops.qkv_rope_append(qkv, 1, L, nq, nkv, hd, Lw.q_norm, Lw.k_norm, eps, inv_freq, cache.seq_lens,
                                     cache.block_table, cache.page, cache.kv_dtype, k_pool, v_pool, k_sb, v_sb)
-            o = ops.attention(q, 1, L, nq, nkv, hd, a.attn_scale, cache.seq_lens, cache.max_ctx, cache.block_table,
+            o = ops.attention(q, 1, L, nq, nkv, hd, a.attn_scale, cache.seq_lens, ctx, cache.block_table,
                               cache.page, cache.kv_dtype, k_pool, v_pool, k_sb, v_sb, causal=True, window=a.window(l))
             h.addmm_(o, rows(l, "o").t())
             ops.rows_rmsnorm(h, Lw.post_norm, eps, out=x)

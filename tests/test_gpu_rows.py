@@ -99,18 +99,7 @@ def test_prepared_rows(dev, M, K):
     assert torch.equal(plain.data.view(Mp // 16, G, 2, 4, 16, 8).permute(0, 4, 1, 3, 2, 5).reshape(Mp, K)[:M], h)
 
 
-@pytest.mark.parametrize("hd,kv_bits,lens,W,nq,nkv,causal,window", [
-    (128, 8, [0], 203, 8, 2, True, 0),            # 64-row blocks
-    (128, None, [5, 700], 1100, 64, 2, True, 0),  # 256-row blocks (G = 32)
-    (128, None, [70], 65, 2, 2, True, 33),
-    (256, None, [0], 1027, 4, 2, True, 0),
-    (256, 8, [900, 3], 65, 8, 8, True, 130),      # windows that start inside a block
-    (256, None, [40], 129, 4, 1, False, 0),
-])
-def test_many_row_attention(dev, hd, kv_bits, lens, W, nq, nkv, causal, window):
-    """Against a float64 softmax over the stored keys: probabilities within 2^-26 and float32 sums
-    leave the output's own bf16 rounding (2^-9) and the queries' and keys' products (float32) well
-    inside 2^-7 of the largest output."""
+def _check_many_rows(dev, hd, kv_bits, lens, W, nq, nkv, causal, window, two_terms=False):
     from mlx_dspark import ops
     from mlx_dspark.kv import PagedKVCache
     print(f"attention rows hd={hd} kv_bits={kv_bits} lens={lens} W={W} window={window}", flush=True)
@@ -133,9 +122,9 @@ def test_many_row_attention(dev, hd, kv_bits, lens, W, nq, nkv, causal, window):
         pools.append(v.view(pool.shape).to(torch.bfloat16).double())
     cache.set_lengths(lens)
     q = torch.randn(B * W, nq * hd, generator=g, device=dev).to(torch.bfloat16)
-    out = ops.attention_rows(q, B, W, nq, nkv, hd, hd ** -0.5, cache.seq_lens, cache.max_ctx, cache.block_table,
-                             cache.page, cache.kv_dtype, *cache.layer_args(0), causal=causal, window=window)
-    got = out.double().view(B, W, nq, hd)
+    outs = [f(q, B, W, nq, nkv, hd, hd ** -0.5, cache.seq_lens, cache.max_ctx, cache.block_table, cache.page,
+              cache.kv_dtype, *cache.layer_args(0), causal=causal, window=window).double().view(B, W, nq, hd)
+            for f in ([ops.attention_rows, ops.attention] if two_terms else [ops.attention_rows])]
     for b, L0 in enumerate(lens):
         n = L0 + W
         K, V = (p[cache.block_table[b].long()].transpose(1, 2).reshape(-1, nkv, hd)[:n] for p in pools)
@@ -147,7 +136,39 @@ def test_many_row_attention(dev, hd, kv_bits, lens, W, nq, nkv, causal, window):
         for t in range(nq):
             sc = (q.double().view(B, W, nq, hd)[b, :, t] @ K[:, t * nkv // nq].T) * hd ** -0.5
             ref = torch.softmax(sc.masked_fill(~ok, -float("inf")), -1) @ V[:, t * nkv // nq]
-            assert float((got[b, :, t] - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())
+            for got in outs:
+                assert float((got[b, :, t] - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("hd,kv_bits,lens,W,nq,nkv,causal,window", [
+    (128, 8, [0], 203, 8, 2, True, 0),            # 64-row blocks
+    (128, None, [5, 700], 1100, 64, 2, True, 0),  # 256-row blocks (G = 32)
+    (128, None, [70], 65, 2, 2, True, 33),
+    (256, None, [0], 1027, 4, 2, True, 0),
+    (256, 8, [900, 3], 65, 8, 8, True, 130),      # windows that start inside a block
+    (256, None, [40], 129, 4, 1, False, 0),
+])
+def test_many_row_attention(dev, hd, kv_bits, lens, W, nq, nkv, causal, window):
+    """Against a float64 softmax over the stored keys: probabilities within 2^-26 and float32 sums
+    leave the output's own bf16 rounding (2^-9) and the queries' and keys' products (float32) well
+    inside 2^-7 of the largest output."""
+    _check_many_rows(dev, hd, kv_bits, lens, W, nq, nkv, causal, window)
+
+
+@pytest.mark.parametrize("kv_bits,lens,W,nq,nkv,causal,window", [
+    (8, [100, 1000, 7], 700, 32, 8, True, 0),      # 256-row blocks: ragged rows, a partial last block
+    (None, [100, 1000, 7], 700, 32, 8, True, 0),
+    (8, [0], 2100, 64, 8, True, 333),              # windows that start inside a key block
+    (None, [0], 2100, 64, 8, True, 333),
+    (8, [50], 1100, 32, 8, False, 0),              # one 64-row block too many for two workgroups per CU
+    (None, [0], 1300, 32, 8, True, 0),             # few cached positions: 64-row blocks past that
+    (8, [900], 1024, 32, 8, True, 0),              # the last size of 64-row blocks, and one row more
+    (8, [900], 1025, 32, 8, True, 0),
+])
+def test_many_row_attention_block_shapes(dev, kv_bits, lens, W, nq, nkv, causal, window):
+    """Both block shapes of head_dim 128 on each side of their rule, with the probabilities as three bf16
+    terms and as two (within 2^-17: the same bound)."""
+    _check_many_rows(dev, 128, kv_bits, lens, W, nq, nkv, causal, window, two_terms=True)
 
 
 def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
