@@ -21,7 +21,8 @@ from ._hip import (DSK_BF16, DSK_EPI_GEGLU, DSK_EPI_PARTIAL, DSK_EPI_RESIDUAL, D
 __all__ = [
     "W8Weight", "W8Table", "Workspace", "Packed", "act_pack", "pack", "pack_rn", "w8_gemm", "w8_residual", "w8_embed",
     "w8_dequant", "Rows", "rows_prep", "w8_rows", "rows_rmsnorm", "rows_gated",
-    "qkv_rope_append", "attention", "attention_rows", "qkv_attention", "row_logprobs", "accept_greedy", "accept_sample", "sample_rows",
+    "qkv_rope_append", "attention", "attention_rows", "attention_rows_split",
+    "qkv_attention", "row_logprobs", "accept_greedy", "accept_sample", "sample_rows",
     "argmax_rows", "lens_add",
     "rope_inv_freq", "DSK_EPI_STORE", "DSK_EPI_SWIGLU", "DSK_EPI_GEGLU", "DSK_EPI_PARTIAL", "DSK_KV_BF16",
     "DSK_KV_U8",
@@ -504,6 +505,26 @@ def attention(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page,
 def attention_rows_takes(hd: int, max_pages: int) -> bool:
     """Whether dsk_attention_rows takes a head_dim and a block table's width."""
     return hd in (128, 256) and max_pages <= ROWS_MAX_PAGES
+
+
+def attention_rows_split(L: int, nq: int, nkv: int, hd: int, cached: int, max_ctx: int, window: int = 0) -> int:
+    """Rows per pass for attention with key splits where that is faster for L new rows after ``cached``
+    positions, 0 where attention_rows is. attention_rows reads its keys one block after the other: few rows
+    leave it few workgroups, each as long as the context is. A split pass takes at most 64 rows (256 or,
+    at head_dim 256, 128 query rows per kv head) and pays its launches and its splits once per pass.
+
+    Times in us of the two, fitted to a sweep over 8 to 32 heads, 0 to 32000 cached positions and 65 to 2048
+    rows (many-row / split, 32 heads of 128 over 8 kv heads, 8-bit: 65 rows after 8000 358 / 77, 255 rows
+    360 / 257, 450 rows 375 / 507, 128 rows after 300 26 / 55); the pick is within a fifth of the better."""
+    if hd not in (128, 256):
+        return 0
+    per = min(64, (256 if hd == 128 else 128) // (nq // nkv))
+    if per == 0:
+        return 0
+    keys = min(cached, window) if window else cached
+    base, key, one, empty, work = (15.0, 0.040, 15.0, 6e-4, 2.3e-6) if hd == 128 else (5.0, 0.085, 24.0, 1.1e-3, 8.4e-6)
+    split = -(-L // per) * (one + empty * max_ctx + work * nkv * (per * (nq // nkv) + 64) * keys)
+    return per if split < base + key * keys else 0
 
 
 def attention_rows(q, B, W, nq, nkv, hd, scale, seq_lens, max_ctx, block_table, page, kv_dtype, k_pool, v_pool,

@@ -353,6 +353,26 @@ class Qwen3W8:
         takes = ops.attention_rows_takes(self.args.head_dim, cache.block_table.shape[1])
         return PREFILL_CHUNK if takes else SPLIT_CHUNK
 
+    def _rows_attention(self, q: torch.Tensor, L: int, window: int, cache: PagedKVCache, l: int,
+                        starts: list) -> torch.Tensor:
+        """Causal attention of _rows_pass's L rows over the cache they were appended to, many rows at a time
+        or, after a long context, with key splits a few rows at a time."""
+        a = self.args
+        nq, nkv, hd = a.num_attention_heads, a.num_key_value_heads, a.head_dim
+        per = 0
+        if ops.attention_rows_takes(hd, cache.block_table.shape[1]):
+            per = ops.attention_rows_split(L, nq, nkv, hd, cache.lengths[0], cache.max_ctx, window)
+        pools = (cache.max_ctx, cache.block_table, cache.page, cache.kv_dtype, *cache.layer_args(l))
+        if per == 0:
+            return ops.attention_rows(q, 1, L, nq, nkv, hd, a.attn_scale, cache.seq_lens, *pools, window=window)
+        if not starts:
+            starts.extend(cache.seq_lens + r for r in range(0, L, per))
+        out = torch.empty((L, nq * hd), dtype=torch.bfloat16, device=q.device)
+        for i, r in enumerate(range(0, L, per)):
+            e = min(L, r + per)
+            ops.attention(q[r:e], 1, e - r, nq, nkv, hd, a.attn_scale, starts[i], *pools, window=window, out=out[r:e])
+        return out
+
     def _rows_pass(self, ids: torch.Tensor, cache: PagedKVCache, tap=None, *, logits: str = "last"):
         """forward over one row of more than MAX_ROWS new tokens, with its rounding points: row-major
         activations between the products of many rows. logits: "last" or "none"; advances the cache.
@@ -364,6 +384,7 @@ class Qwen3W8:
         tap = list(tap or [])
         h = self.embed_rows(ids.reshape(-1))
         fused = torch.empty((L, len(tap) * H), dtype=torch.bfloat16, device=self.device) if tap else None
+        starts: list = []   # seq_lens at each split pass's first row, once for all layers
         x = ops.rows_prep(h, norm_w=self.layers[0].in_norm, eps=eps, later=not sandwich)
         for l, Lw in enumerate(self.layers):
             slots = [i for i, t in enumerate(tap) if t == l]
@@ -375,9 +396,7 @@ class Qwen3W8:
             q = ops.qkv_rope_append(ops.w8_rows(x, Lw.qkv), 1, L, nq, nkv, hd, Lw.q_norm, Lw.k_norm, eps, inv_freq,
                                     cache.seq_lens, cache.block_table, cache.page, cache.kv_dtype, k_pool, v_pool,
                                     k_sb, v_sb)
-            o = ops.attention_rows(q, 1, L, nq, nkv, hd, a.attn_scale, cache.seq_lens, cache.max_ctx,
-                                   cache.block_table, cache.page, cache.kv_dtype, k_pool, v_pool, k_sb, v_sb,
-                                   causal=True, window=a.window(l))
+            o = self._rows_attention(q, L, a.window(l), cache, l, starts)
             o = ops.rows_prep(o)
             if sandwich:
                 y = ops.w8_rows(o, Lw.o)

@@ -192,6 +192,36 @@ def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
         assert float((a.float() - b.float()).abs().max()) <= 2e-2 * float(b.float().abs().max())
 
 
+@pytest.mark.parametrize("name,n", [("tiny-gemma", 70), ("tiny-gemma", 200), ("tiny", 65), ("tiny", 130)])
+def test_prompt_after_a_long_context_equals_forward_passes(dev, monkeypatch, name, n):
+    """A second turn: few rows after many cached positions take the key-split attention (of the Gemma-style
+    layers, the global one only). The taps and logits of 64-row forward passes, up to rounding flips."""
+    from mlx_dspark import ops, synthetic
+    model = synthetic.build_target(name, seed=45)
+    a, cached = model.args, 6000
+    prompt = torch.randint(0, a.vocab_size, (n,), generator=torch.Generator().manual_seed(3)).tolist()
+    passes, real = [], ops.attention
+    monkeypatch.setattr(ops, "attention", lambda q, B, W, *r, **k: (passes.append(W), real(q, B, W, *r, **k))[1])
+    g = torch.Generator(device=dev).manual_seed(9)
+    pools = [[torch.randn(p.shape, generator=g, device=dev).to(p.dtype) for p in pool]
+             for pool in (lambda c: (c.k, c.v))(model.make_cache(max_ctx=cached + n))]
+    outs = []
+    for chunk in (64, 63):           # 63: forward passes
+        cache = model.make_cache(max_ctx=cached + n)
+        for pool, src in zip((cache.k, cache.v), pools):
+            for p, x in zip(pool, src):
+                p.copy_(x)
+        cache.set_lengths([cached])
+        passes.clear()
+        logits, fused = model.prefill(prompt, cache, [0, a.num_hidden_layers - 1], chunk=chunk)
+        if chunk == 64:
+            split = a.num_hidden_layers if name == "tiny" else 1
+            assert sorted(passes) == sorted([min(64, n - r) for r in range(0, n, 64)] * split)
+        outs.append((logits, fused, cache.k[-1], cache.v[-1]))
+    for x, y in zip(*outs):
+        assert float((x.float() - y.float()).abs().max()) <= 2e-2 * float(y.float().abs().max())
+
+
 def test_prompt_pieces_wider_than_a_forward_pass_are_refused(dev):
     """An explicit chunk of more than 64 rows, before any key is appended; a prompt that fits one pass is
     taken whatever the chunk."""
