@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kPrepThreads) void rows_prep_kernel(PrepArgs a) {
     s += __shfl_xor(s, 1, 64);  // 8 neighbouring threads hold one group
     s += __shfl_xor(s, 2, 64);
     s += __shfl_xor(s, 4, 64);
-    if ((tid & 7) == 0 && g < a.Gp) {
+    if ((tid & 7) == 0 && g < a.Gp) {  // the NV kPrepThreads chunks cover Gp: padding groups get zero
       const Bf16x2Terms t = split3_bf16x2(live ? s : 0.0f, 0.0f);
       const int64_t o = rows_index(m, g, a.Gp / 64);
       a.xt[o] = (uint16_t)(t.hi & 0xffffu);
@@ -153,10 +153,6 @@ __global__ __launch_bounds__(kPrepThreads) void rows_prep_kernel(PrepArgs a) {
       a.xt[2 * a.plane + o] = (uint16_t)(t.lo & 0xffffu);
     }
   }
-  // padding groups past the chunks above are zero
-  if (a.x)
-    for (int64_t g = (int64_t)NV * kPrepThreads / 8 + tid; g < a.Gp; g += kPrepThreads)
-      for (int p = 0; p < 3; ++p) a.xt[p * a.plane + rows_index(m, g, a.Gp / 64)] = 0;
 }
 
 // =====================================================================================

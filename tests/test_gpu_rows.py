@@ -60,14 +60,18 @@ def test_products_of_many_rows(dev, M, N, K, bits):
     if N % 32:
         return
     Wp, w64, mag = _weight(N, K, bits, True, dev)
-    ref = (x64 @ w64.T) * r
+    ref, bound = (x64 @ w64.T) * r, K * 2.0 ** -24 * (x64.abs() @ mag.T) * r
+    e_gate, e_up = (bound + 2.0 ** -8 * ref.abs()).split(N // 2, dim=1)   # each rounded to bf16
     gate, up = ref[:, :N // 2], ref[:, N // 2:]
     for epi, act in ((DSK_EPI_SWIGLU, torch.nn.functional.silu(gate)),
                      (DSK_EPI_GEGLU, torch.nn.functional.gelu(gate, approximate="tanh"))):
         y, want = w8_rows(x, Wp, epi=epi), act * up
         # three bf16 roundings (gate, up, act) of factors of at most slope 1.13, and the store's
-        err = (y.double() - want).abs() - 2.0 ** -6 * ((gate.abs() + act.abs()) * up.abs())
-        assert float(err.max()) <= float(bound.max()) * float(ref.abs().max()) * 4
+        # element by element: the gate's error through the activation (slope at most 1.13) and its rounding,
+        # times up, up's times the activation, and the store's rounding
+        e_act = 1.13 * e_gate + 2.0 ** -8 * act.abs()
+        assert bool(((y.double() - want).abs() <= act.abs() * e_up + e_act * (up.abs() + e_up)
+                     + 2.0 ** -8 * want.abs()).all())
 
 
 @pytest.mark.parametrize("M,K", [(1, 64), (3, 4096), (67, 4160), (130, 12288), (5, 24576)])
@@ -169,6 +173,45 @@ def test_many_row_attention_block_shapes(dev, kv_bits, lens, W, nq, nkv, causal,
     """Both block shapes of head_dim 128 on each side of their rule, with the probabilities as three bf16
     terms and as two (within 2^-17: the same bound)."""
     _check_many_rows(dev, 128, kv_bits, lens, W, nq, nkv, causal, window, two_terms=True)
+
+
+@pytest.mark.parametrize("hd,W", [(128, 65), (128, 4200), (256, 65)])
+def test_probabilities_carry_three_terms(dev, hd, W):
+    """Values that cancel leave the probabilities' own error: five keys with weights of e^-1.2 to 1, the last
+    two values chosen so that every output is below 2^-14 of the weighted magnitudes sum(p |v|) and its bf16
+    store hides nothing above 2^-23 of them. Float32 probabilities (exp2 and its argument within 2^-22) and
+    sums stay within 2^-21; two bf16 terms, each weight off by up to 2^-17, do not (dsk_attention, head_dim
+    128). At 4200 rows the 256-row blocks run."""
+    from mlx_dspark import ops
+    from mlx_dspark.kv import PagedKVCache
+    n = 8
+    cache = PagedKVCache(1, 1, n, hd, W)
+    g = torch.Generator(device=dev).manual_seed(hd + W)
+    # keys 0-4 of head h: q . k = 8 a[h, j], exact in bf16; the others' weights vanish
+    a = torch.zeros(n, 5)
+    a[:, 1:] = -torch.rand(n, 4, generator=torch.Generator().manual_seed(hd)) * 1.2 * hd ** 0.5 / 8
+    a = a.to(torch.bfloat16).to(dev)
+    K = torch.zeros(n, cache.max_ctx, hd, dtype=torch.bfloat16, device=dev)
+    K[:, :, 0] = -200.0
+    K[:, :5, 0] = a
+    p = torch.softmax(8 * a.double() * float(torch.tensor(hd ** -0.5)), 1)          # [n, 5]
+    V = torch.zeros(n, cache.max_ctx, hd, dtype=torch.bfloat16, device=dev)
+    V[:, :3] = torch.randn(n, 3, hd, generator=g, device=dev).to(torch.bfloat16)
+    for j in (3, 4):
+        V[:, j] = (-(p[:, :j, None] * V[:, :j].double()).sum(1) / p[:, j, None]).to(torch.bfloat16)
+    for pool, x in ((cache.k[0], K), (cache.v[0], V)):
+        pool.copy_(x.view(n, cache.max_pages, 64, hd).transpose(0, 1))
+    q = torch.zeros(W, n, hd, dtype=torch.bfloat16, device=dev)
+    q[:, :, 0] = 8.0
+    ref = (p[..., None] * V[:, :5].double()).sum(1)
+    size = (p[..., None] * V[:, :5].double().abs()).sum(1)
+    assert bool((ref.abs() <= 2.0 ** -14 * size).all())
+    args = (q.view(W, -1), 1, W, n, n, hd, hd ** -0.5, cache.seq_lens, cache.max_ctx, cache.block_table, cache.page,
+            cache.kv_dtype, *cache.layer_args(0))
+    err = lambda out: float(((out.double().view(W, n, hd) - ref).abs() / size).max())
+    assert err(ops.attention_rows(*args, causal=False)) <= 2.0 ** -21
+    if hd == 128:
+        assert err(ops.attention(*args, causal=False)) > 2.0 ** -20
 
 
 def test_prompt_longer_than_a_piece_equals_forward_passes(dev):
