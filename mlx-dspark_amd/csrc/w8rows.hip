@@ -13,7 +13,7 @@
 // that precedes it (with the sandwich norm), the RMSNorm, the X terms, and x in the order the product's
 // loads take it (rows_index): one wave-wide load of an MFMA operand is 1 KiB of consecutive bytes. Read
 // from row-major rows the 64 lanes of a load touch 64 separate pieces of 16 bytes (lanes next to each
-// other hold different rows), and the product took 832 us against 462 (24576 x 4096, 2048 rows).
+// other hold different rows), and the product took 1.8 times as long (24576 x 4096, 2048 rows).
 #include "common.h"
 #include "wfrag.h"
 
@@ -193,16 +193,17 @@ __device__ __forceinline__ void codes_to_bf16(const u32x2 w, bf16x8& lo, bf16x8&
 // A workgroup computes 64 MTW rows x 16 NTW columns: its four waves own 16 MTW rows each and share
 // every code, which one of them converts to bf16 and leaves in LDS (two buffers, one barrier per U
 // 64-column groups; codes are loaded two steps ahead, the rows of x one, straight into the registers
-// that feed the MFMA). KS > 1: KS such sets of four waves take a slice of the groups each. The weights are the A operand, so a lane ends with four consecutive columns of
-// one row. Workgroup ids: a column block's row blocks run one after the other on one XCD, whose L2
-// then holds the column block's codes.
+// that feed the MFMA). KS > 1: KS such sets of four waves take a slice of the groups each. The weights are
+// the A operand, so a lane ends with four consecutive columns of one row. Workgroup ids: a column block's
+// row blocks run one after the other on one XCD, whose L2 then holds the column block's codes.
 //
-// What bounds it: with 256 x 64 tiles the 24576 x 4096 gate_up over 2048 rows takes 495 us = 833 TFLOP/s
-// (o 4096 x 4096 79 us, 870). Working copies without the loads of x, the scaling or the conversion of
-// the codes took 0.63, 0.75 and 0.71 of the time, without all three 0.43: the matrix pipe alone would
-// reach 1.65 PFLOP/s behind the barriers, and the L2 traffic of x (6.4 GB) and the VALU work each add
-// to it. Sharing x between two column halves of eight waves, 256 x 128 tiles or more steps in flight
-// measured no faster.
+// What bounds it: with 256 x 64 tiles the 24576 x 4096 gate_up over 2048 rows takes 485 us = 849 TFLOP/s
+// (stored without its activation 473; o 4096 x 4096 89 us, 771). Working copies of the 473 us without the
+// loads of x or the scaling took 0.71 and 0.84 of it, without the conversion of the codes as long, without
+// all three 0.58: the matrix pipe alone would reach 1.5 PFLOP/s behind the barriers, and the L2 traffic of x
+// (6.4 GB) and the scaling's VALU work each add to it. Sharing x between two column halves of eight waves,
+// 256 x 128 tiles or more steps in flight measured no faster at 2048 rows; at 1027, where 128-row tiles run,
+// two column halves of them took 271 against 288 us (not built).
 template <int MTW, int NTW, int U, int KS, int BITS, int EK>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS < 2 ? 2 : KS))) void w8_rows_kernel(RowsArgs a) {
   using WT = typename WeightChunk<BITS>::type;
@@ -443,8 +444,8 @@ struct RowsPlan {
 
 // A sweep on MI355X over the Qwen3-8B and Gemma-style 12B projections (and the 4-bit DFlash context's)
 // at M = 65, 130, 203, 300, 700, 1027 and 2048 (times in us):
-//  - 256 x 64 where that gives every CU two workgroups (gate_up 24576 x 4096 at M = 2048: 495 against
-//    547 for 128 x 64; its four waves read 8 KB of x per group for 32 MFMAs each) and its last row
+//  - 256 x 64 where that gives every CU two workgroups (gate_up 24576 x 4096 at M = 2048: 496 against
+//    537 for 128 x 64; its four waves read 8 KB of x per group for 32 MFMAs each) and its last row
 //    block pads the rows by no more than the 128-row one would by a tenth;
 //  - else 128 x 64 with the groups in one slice from 512 workgroups (o 4096 x 4096 at M = 1027: 62),
 //    two from 256 (o at M = 700: 43 against 48 in one slice), four above 128 (qkv 6144 x 4096 at
