@@ -266,7 +266,8 @@ int dsk_qkv_norm_rope_append(const void* qkv, int qkv_splits, int B, int W, int 
  * causal == 0: every query sees all seq_lens[b] + W keys (DSpark/DFlash block attention,
  *   src/mlx_dspark/model.py:130-155, dflash_model.py:123-133).
  * q [B*W, nq*hd] bf16 -> out [B*W, nq*hd] bf16. GQA: q head h reads kv head h/(nq/nkv).
- * max_ctx bounds seq_lens[b] + W (sizes the split grid so the launch is graph-stable).
+ * max_ctx bounds seq_lens[b] + W (sizes the split grid so the launch is graph-stable; the many-query
+ * form chooses its query blocks by it).
  * softcap > 0: scores = tanh(scores / softcap) * softcap before the mask.
  * out_packed != 0 writes the output in the packed activation layout (the o-projection's x).
  * Probabilities stay float32: the P.V products run as three bf16 MFMAs over P's hi + mid + lo
