@@ -472,10 +472,10 @@ class Qwen3W8:
         qkv = torch.empty((L, a.n_qkv), dtype=torch.bfloat16, device=dev)
         gu = torch.empty((L, 2 * I), dtype=torch.bfloat16, device=dev)
         act = torch.empty((L, I), dtype=torch.bfloat16, device=dev)
-        # the many-query kernel takes max_ctx as a bound of the keys only to choose its blocks; the
-        # split one (other head_dims, very long caches) sizes its splits by it
-        bounded = hd == 128 and ops.attention_rows_takes(hd, cache.block_table.shape[1])
-        ctx = cache.lengths[0] + L if bounded else cache.max_ctx
+        # the many-query kernel takes max_ctx as a bound of the keys only to choose its blocks; the split
+        # ones (up to MAX_ROWS rows, other head_dims, very long caches) size their splits by it
+        many = L > MAX_ROWS and hd == 128 and ops.attention_rows_takes(hd, cache.block_table.shape[1])
+        ctx = cache.lengths[0] + L if many else cache.max_ctx
         for l, Lw in enumerate(self.layers):
             ops.rows_rmsnorm(h, Lw.in_norm, eps, out=x)
             torch.matmul(x, rows(l, "qkv").t(), out=qkv)
